@@ -349,6 +349,31 @@ int wkv_prefill_gqa_sinks(const wkv_cache_t *cache, const void *key, int64_t key
                           const int32_t *block_table, int64_t bt_stride, int32_t max_blocks_per_seq, int32_t batch,
                           int32_t max_query_len, int32_t max_seq_len, float scale, const float *sinks, void *stream);
 
+/* wkv_prefill_gqa with a workspace, so that a launch with too few query tiles
+ * for the chip (a few new tokens over a long context) can share its keys
+ * evenly over the chip's workgroups: a query tile whose keys fall to several
+ * workgroups leaves fp32 partials in the workspace and a second kernel merges
+ * them by log-sum-exp. Otherwise the arguments, result and behaviour of
+ * wkv_prefill_gqa (of wkv_prefill_gqa_sinks with sinks non-NULL).
+ * workgroups: 0 = the library's choice (sharing only where it is expected to
+ * be faster), n > 0 = share over n (rounded up to a multiple of 8; ignored for
+ * launches of more than 1,024 groups of four 32-query tiles per KV head).
+ * workspace: wkv_prefill_workspace_size() bytes for the same geometry and
+ * workgroups, max_seq_len clipped to the block-table width (0 bytes = nothing
+ * is shared; workspace may then be NULL). No counterpart in the reference
+ * beyond wkv_prefill_gqa's. */
+int64_t wkv_prefill_workspace_size(int32_t batch, int32_t kv_dtype, int32_t num_kv_heads, int32_t num_q_heads,
+                                   int32_t head_dim, int32_t max_query_len, int32_t max_seq_len, int32_t workgroups);
+
+int wkv_prefill_gqa_shared(const wkv_cache_t *cache, const void *key, int64_t key_stride_t, int64_t key_stride_h,
+                           const void *value, int64_t value_stride_t, int64_t value_stride_h,
+                           const int64_t *slot_mapping, int64_t num_tokens, const void *q, int64_t q_stride_t,
+                           int64_t q_stride_h, void *out, int64_t out_stride_t, int64_t out_stride_h,
+                           int32_t num_q_heads, const int32_t *cu_seqlens_q, const int32_t *seq_lens,
+                           const int32_t *block_table, int64_t bt_stride, int32_t max_blocks_per_seq, int32_t batch,
+                           int32_t max_query_len, int32_t max_seq_len, float scale, int32_t workgroups,
+                           void *workspace, int64_t workspace_bytes, const float *sinks, void *stream);
+
 /* Token sampler: the step after decode, producing what the engine records per
  * generated token -- the token, its processed logprob and the sampling mask
  * (llm.generate with logprobs_mode="processed_logprobs" and

@@ -16,9 +16,11 @@ import ctypes
 import torch
 
 from . import _lib
-from .cache import MLALatentCache, PagedKVCache, _require_cuda, _slots, _stream, _token_rows, check_tables
+from .cache import KV_DTYPES, MLALatentCache, PagedKVCache, _require_cuda, _slots, _stream, _token_rows, check_tables
 
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
+
+_SHARE_MIN_KEYS = 1024  # the library shares no prefill launch over fewer keys (kShareMinKeys)
 
 
 def _key(device: torch.device) -> tuple[int, int]:
@@ -365,8 +367,20 @@ def prefill_gqa(
     args = (ctypes.byref(cache.descriptor()), *head, q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(),
             out.stride(0), out.stride(1), hq, cu_seqlens_q.data_ptr(), seq_lens.data_ptr(), block_table.data_ptr(),
             block_table.stride(0), block_table.shape[1], batch, int(max_query_len), msl, float(scale))
-    if sinks is not None:
-        rc = lib.wkv_prefill_gqa_sinks(*args, sinks.data_ptr(), _stream(dev))
+    # scratch for a small grid's shared key ranges (none for most prompts, and never up to
+    # _SHARE_MIN_KEYS keys); from the caching allocator on the call's own stream, so it needs
+    # no owner across streams, threads or captures
+    keys = min(msl, block_table.shape[1] * cache.block_size)
+    need = 0
+    if keys > _SHARE_MIN_KEYS and batch:
+        need = lib.wkv_prefill_workspace_size(batch, KV_DTYPES[cache.kv_dtype], cache.num_kv_heads, hq, cache.head_dim,
+                                              int(max_query_len), keys, 0)
+    sinks_ptr = sinks.data_ptr() if sinks is not None else None
+    if need > 0:
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        rc = lib.wkv_prefill_gqa_shared(*args, 0, ws.data_ptr(), need, sinks_ptr, _stream(dev))
+    elif sinks is not None:
+        rc = lib.wkv_prefill_gqa_sinks(*args, sinks_ptr, _stream(dev))
     else:
         rc = lib.wkv_prefill_gqa(*args, _stream(dev))
     _lib.check(rc, "prefill_gqa")

@@ -7,20 +7,26 @@
 // aligned mask of a varlen prefill over a paged context (a prefix-cache hit or
 // an earlier chunk).
 //
-// Work decomposition: workgroup (query tile, KV head x head group, sequence)
-// of four waves; wave w takes query head kvh*G + 4*hg + w, so the MFMA
-// columns are consecutive query tokens of one head and the four waves of a
-// workgroup stream the same key tiles. Every query tile of a (sequence, KV
-// head) re-reads that head's keys, so the 1-D grid sends all of them to one
-// XCD (the dispatcher deals workgroup i to XCD i mod 8): the keys are served
-// from that XCD's L2 instead of being fetched by all eight. The latest (most
-// expensive, causally) query tiles are dispatched first. Keys are copied once
-// per workgroup into LDS by LDS-DMA, in 16-token tiles, four per step of 64
-// keys; each wave holds 32 queries and runs 32x32x16 bf16 MFMAs. fp8 tiles
-// are dequantized in LDS (exactly: power-of-two scales) by the wave that
-// copied them, so both dtypes share the attention arithmetic. Tiles on the
-// causal diagonal mask per lane (column). Every wave finishes its rows: no
-// split-K, no workspace.
+// Work decomposition: the query rows of one (sequence, KV head) are units of
+// one query head x 32 consecutive query tokens, unit u = tile u / G of head
+// u % G; a workgroup of four waves takes four consecutive units, one per wave,
+// so the MFMA columns are consecutive query tokens of one head and the four
+// waves stream the same key tiles. Units run over head and tile together, so
+// no wave idles when G is not a multiple of four (G = 7: 7/8 of the waves
+// worked when a workgroup held four heads of one tile; G = 2: half of them).
+// Every unit group of a (sequence, KV head) re-reads that head's keys, so the
+// 1-D grid sends them to one XCD (the dispatcher deals workgroup i to XCD
+// i mod 8): the keys are served from that XCD's L2 instead of being fetched by
+// all eight. The latest (most expensive, causally) query tiles are dispatched
+// first. Keys are copied once per workgroup into LDS by LDS-DMA, in 16-token
+// tiles, four per step of 64 keys; each wave holds 32 queries and runs
+// 32x32x16 bf16 MFMAs. fp8 tiles are dequantized in LDS (exactly:
+// power-of-two scales) by the wave that copied them, so both dtypes share the
+// attention arithmetic. Tiles on the causal diagonal mask per lane (column).
+// A grid too small for the chip (a few new tokens over a long context) shares
+// its 64-key steps evenly over a fixed number of workgroups instead
+// (prefill_grid): a workgroup's share may end inside a unit group, whose parts
+// leave fp32 partials that prefill_merge_kernel combines by log-sum-exp.
 #include "gqa_tiles.h"
 #include "lds_dma.h"
 
@@ -29,6 +35,18 @@
 namespace wkv {
 
 constexpr int kPrefillWaves = 4;
+// The rule that shares a launch's steps over a fixed number of workgroups
+// (prefill_grid) compares two estimates in microseconds, fitted to launches of
+// 16 to 376 unit groups over 500 to 15,000 keys (bf16, d=128):
+constexpr int kPrefillCus = 256;
+constexpr int kShareMinKeys = 1024;   // below, no estimate favours sharing (its second launch alone costs the gain)
+constexpr double kStepUs = 1.08;      // one 64-key step of a workgroup alone on its CU, bf16
+constexpr double kStepFp8Us = 1.45;   // ... fp8 (the conversion stands before the barrier)
+constexpr double kStepPairUs = 2.0;   // a step of each of two on a CU, either type
+constexpr double kPartUs = 0.05;      // writing and merging a workgroup's partials
+constexpr double kGroupUs = 6.0;      // starting a unit group (its queries, table and first keys)
+constexpr double kLaunchUs = 5.0;     // a plain launch's fixed part
+constexpr double kShareUs = 9.5;      // a shared launch's: with the prefix and the merge's launch
 
 // Eight e4m3fn codes (bytes of lo, then hi) times a power-of-two scale as
 // eight bf16 values, by the hardware pair conversion (exact: every such
@@ -94,14 +112,160 @@ struct LdsTile {
 // bf16) after the wait and before the barrier of the step: its V tile of
 // step s and its K tile of step s + 1. The attention arithmetic is the bf16
 // one. LDS: 64 KB bf16 plus 8 + 8 KB staging at d=128.
-template <int D, bool FP8>
-__global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(
-    const uint8_t *__restrict__ kc, const uint8_t *__restrict__ vc, const float *__restrict__ ksc,
-    const float *__restrict__ vsc, const uint16_t *__restrict__ q, int64_t q_st,
-    int64_t q_sh, uint16_t *__restrict__ out, int64_t o_st, int64_t o_sh, const int32_t *__restrict__ cu_q,
-    const int32_t *__restrict__ seq_lens, const int32_t *__restrict__ bt, int64_t bt_stride, int Mb, int max_seq,
-    int Hkv, int G, int n_hg, int BS, int nb, float scale_log2, int n_qt, int n_items,
-    const float *__restrict__ sinks) {
+// Division of a non-negative int by a divisor known on the host, in a handful
+// of scalar instructions (a runtime division takes some 40 vector ones, and
+// half a dozen of them stood in a row before a workgroup's first load: a
+// 60-token prompt's launch 8.5 us, 8.0 without them). m = min(floor(2^32 / d), 2^32 - 1) gives a quotient at
+// most one too small for every x below 2^31.
+struct FastDiv {
+  uint32_t m;
+  int d;
+};
+
+static FastDiv fast_div(int d) {
+  return FastDiv{d == 1 ? 0xffffffffu : static_cast<uint32_t>((1ull << 32) / static_cast<uint32_t>(d)), d};
+}
+
+__device__ __forceinline__ int operator/(int x, const FastDiv &f) {
+  const int q = static_cast<int>(__umulhi(static_cast<uint32_t>(x), f.m));
+  return q + (x - q * f.d >= f.d ? 1 : 0);
+}
+
+// How a launch covers its work (prefill_grid, on the host).
+struct PrefillGrid {
+  int n_ug;     // unit groups (four units) per (sequence, KV head), at the longest query
+  int R;        // XCDs the unit groups of one (sequence, KV head) are dealt over
+  int n_inner;  // workgroups of one (sequence, KV head) per XCD
+  int n_sub;    // (sequence, KV head) x R
+  int W;        // workgroups that share the steps evenly; 0: a workgroup per unit group
+  int batch;
+  int log2R;
+  FastDiv by_G, by_ug, by_inner, by_Hkv;  // query heads per KV head, n_ug, n_inner, KV heads
+};
+
+// The units and 64-key steps of unit group ug of a sequence (uniform).
+struct PrefillRange {
+  int units;    // query heads x query tiles of 32 of the sequence
+  int kend;     // keys [0, kend) of the group's last query
+  int n_steps;  // 64-key steps over them
+};
+
+__device__ __forceinline__ PrefillRange prefill_range(int qlen, int L, const FastDiv &G, int ug) {
+  PrefillRange r;
+  r.units = qlen > 0 ? ((qlen + 31) >> 5) * G.d : 0;
+  int u_last = 4 * ug + 3;
+  u_last = u_last < r.units ? u_last : r.units - 1;
+  const int t_last = u_last >= 0 ? 32 * (u_last / G) : 0;
+  const int last = (t_last + 32 < qlen ? t_last + 32 : qlen) - 1;
+  r.kend = L - qlen + last + 1;
+  r.n_steps = r.kend > 0 ? (r.kend + 63) >> 6 : 0;
+  return r;
+}
+
+// Shared launches. The steps of every unit group in the order (KV head,
+// sequence, unit group) form one line of T steps (a group without keys counts
+// one: its rows are written all the same), and workgroup w takes steps
+// [w T / W, (w + 1) T / W): every workgroup works equally long whatever the
+// mix of lengths, and at most its first and last unit groups are partial.
+// pfx[i] (LDS) is the line's prefix at entry i = sequence * n_ug + group of
+// one KV head, entries in order, pfx[E] their total; every workgroup forms it
+// itself from the lengths (a launch of its own would cost more).
+constexpr int kPrefillEntries = 1024;  // at most this many entries per KV head
+
+__device__ __forceinline__ int prefill_prefix(int *pfx, int *red, const int32_t *cu_q, const int32_t *seq_lens,
+                                              int max_seq, const PrefillGrid &pg) {
+  const int E = pg.batch * pg.n_ug;
+  const int per = (E + 64 * kPrefillWaves - 1) / (64 * kPrefillWaves);  // <= 4 entries per thread
+  const int e0 = threadIdx.x * per;
+  int c[kPrefillEntries / (64 * kPrefillWaves)], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kPrefillEntries / (64 * kPrefillWaves); ++k) {
+    c[k] = 0;
+    const int e = e0 + k;
+    if (k < per && e < E) {
+      const int b = e / pg.by_ug, ug = e - b * pg.n_ug;
+      const int qlen = cu_q[b + 1] - cu_q[b];
+      int L = seq_lens[b];
+      L = L < max_seq ? L : max_seq;
+      const PrefillRange r = prefill_range(qlen, L, pg.by_G, ug);
+      if (4 * ug < r.units) c[k] = r.n_steps > 0 ? r.n_steps : 1;
+    }
+    sum += c[k];
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += y;
+  }
+  if (lane == 63) red[wave] = incl;
+  __syncthreads();
+  int base = incl - sum, total = 0;
+#pragma unroll
+  for (int w = 0; w < kPrefillWaves; ++w) {
+    if (w < wave) base += red[w];
+    total += red[w];
+  }
+#pragma unroll
+  for (int k = 0; k < kPrefillEntries / (64 * kPrefillWaves); ++k)
+    if (k < per && e0 + k < E) {
+      pfx[e0 + k] = base;
+      base += c[k];
+    }
+  if (threadIdx.x == 0) pfx[E] = total;
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(total);
+}
+
+// First step of workgroup w's share of T steps over W workgroups (the callers
+// take W <= T, so that every share has a step: a part's slot is then written
+// by its workgroup whenever the merge reads it).
+__device__ __forceinline__ int64_t prefill_share(int w, int64_t T, int W) { return w * T / W; }
+
+// A part's partial of one unit: D/32 x 4 runs of 64 lanes x 4 fp32 (the
+// output accumulators as the lanes hold them, so both the store and the
+// merge's load are whole 1 KB wave accesses), then the 32 queries' reference
+// maxima (log2 domain) and sums. Workgroup w owns partial slots 2 w (its first
+// unit group) and 2 w + 1 (a later one), four units each.
+template <int D>
+constexpr int prefill_part_floats() {
+  return 32 * D + 64;
+}
+
+// The attention kernel's arguments: one struct, the kernel's only parameter
+// (prefill_args reads it from the kernel-argument segment).
+struct PrefillArgs {
+  const uint8_t *kc, *vc;
+  const float *ksc, *vsc;
+  const uint16_t *q;
+  int64_t q_st, q_sh;
+  uint16_t *out;
+  int64_t o_st, o_sh;
+  const int32_t *cu_q, *seq_lens, *bt;
+  int64_t bt_stride;
+  int Mb, max_seq, Hkv, BS, nb;
+  float scale_log2;
+  FastDiv by_BS;
+  PrefillGrid pg;
+  float *part;
+  const float *sinks;
+};
+
+// The kernel's arguments, read again from the kernel-argument segment (the
+// pointer is opaque to the compiler). A shared launch's loop over unit groups
+// calls this per group: with the arguments live across the loop instead, some
+// 70 scalar registers spill into the key loop (a 64-key step then takes 1.39
+// us against 0.99).
+__device__ __forceinline__ const PrefillArgs &prefill_args() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const PrefillArgs *)(p);
+}
+
+// SHARED: workgroups share the launch's steps evenly (PrefillGrid::W), else one per unit group.
+template <int D, bool FP8, bool SHARED>
+__global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(PrefillArgs kernel_args) {
   using LT = LdsTile<D>;
   static_assert(kPrefillWaves == 4, "one tile per wave per 64-key step");
   static_assert(D % 64 == 0, "whole copies per lane");
@@ -114,34 +278,96 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(
   __shared__ __attribute__((aligned(16))) uint8_t ldsv[2 * 4 * VB];  // bf16 V: two step slots
   __shared__ __attribute__((aligned(16))) uint8_t stgk[4 * SB];      // fp8 K as copied, a tile per wave
   __shared__ __attribute__((aligned(16))) uint8_t stgv[4 * SB];      // fp8 V as copied
-  const int id = blockIdx.x;
-  const int item = (id / (8 * n_qt)) * 8 + (id & 7);
-  const int qt = __builtin_amdgcn_readfirstlane(n_qt - 1 - (id / 8) % n_qt);
-  if (item >= n_items) return;
-  const int b = __builtin_amdgcn_readfirstlane(item / (Hkv * n_hg));
-  const int kvh = __builtin_amdgcn_readfirstlane((item / n_hg) % Hkv);
-  const int hg = item % n_hg;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, n = lane & 31, hh = lane >> 5;
-  const int q0 = cu_q[b];
-  const int qlen = cu_q[b + 1] - q0;
-  int L = seq_lens[b];
-  L = L < max_seq ? L : max_seq;
+  int id = blockIdx.x;
+  // One argument of every 64-byte line, together: the lines come from memory in
+  // one round trip, and the later argument reads hit the scalar cache (taken as
+  // they are needed, the lines' misses stand one after another before the
+  // first load of the queries).
+  // (not volatile: that would count as a write, and loads after it as vector loads)
+  asm("" : "+s"(id) : "s"(kernel_args.kc), "s"(kernel_args.o_sh), "s"(kernel_args.pg.n_ug), "s"(kernel_args.sinks));
+  int b, kvh, ug, s_begin = 0, seg = 0;
+  int64_t steps_left = 0;  // SHARED: of this workgroup's share
+  if constexpr (SHARED) {
+    const PrefillArgs &a = prefill_args();
+    const PrefillGrid pg = a.pg;
+    // XCD i mod 8 takes a contiguous eighth of the line: its workgroups read the same keys.
+    const int w = (id & 7) * (pg.W / 8) + id / 8;
+    int *pfx = reinterpret_cast<int *>(ldsk);
+    static_assert((kPrefillEntries + 1 + kPrefillWaves) * 4 <= 2 * 4 * KB, "the prefix fits the K slots");
+    const int E = pg.batch * pg.n_ug;
+    const int total = prefill_prefix(pfx, pfx + kPrefillEntries + 1, a.cu_q, a.seq_lens, a.max_seq, pg);
+    const int64_t T = static_cast<int64_t>(total) * a.Hkv;
+    const int W = T < pg.W ? static_cast<int>(T) : pg.W;
+    if (w >= W) return;
+    const int64_t x0 = prefill_share(w, T, W);
+    steps_left = prefill_share(w + 1, T, W) - x0;
+    kvh = static_cast<int>(x0 / total);
+    const int y = static_cast<int>(x0 - static_cast<int64_t>(kvh) * total);
+    int lo = 0, hi = E;  // the last entry with pfx <= y (entries of no steps share their successor's prefix)
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (pfx[mid] <= y) lo = mid; else hi = mid;
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    s_begin = __builtin_amdgcn_readfirstlane(y - pfx[lo]);
+    b = lo / pg.by_ug;
+    ug = lo - b * pg.n_ug;
+  } else {
+    const PrefillGrid &pg = kernel_args.pg;
+    // Eight sub-items (item, share r of its unit groups) run at a time, one per XCD.
+    const int oct = (id >> 3) / pg.by_inner;
+    const int inner = (id >> 3) - oct * pg.n_inner;
+    const int sub = 8 * oct + (id & 7);
+    if (sub >= pg.n_sub) return;
+    const int item = sub >> pg.log2R;
+    ug = pg.n_ug - 1 - ((inner << pg.log2R) + (sub & (pg.R - 1)));
+    if (ug < 0) return;
+    b = item / pg.by_Hkv;
+    kvh = item - b * pg.by_Hkv.d;
+  }
+  for (;;) {  // SHARED: the unit groups of the share; else one
+  const PrefillArgs *ap = &kernel_args;
+  if constexpr (SHARED) ap = &prefill_args();
+  const uint8_t *__restrict__ const kc = ap->kc, *__restrict__ const vc = ap->vc;
+  const float *__restrict__ const ksc = ap->ksc, *__restrict__ const vsc = ap->vsc;
+  const int32_t *__restrict__ const cu_q = ap->cu_q;
+  const FastDiv G = ap->pg.by_G;
+  const int Hkv = ap->Hkv, BS = ap->BS, Mb = ap->Mb, nb = ap->nb;
+  const float scale_log2 = ap->scale_log2;
+  b = __builtin_amdgcn_readfirstlane(b);
+  kvh = __builtin_amdgcn_readfirstlane(kvh);
+  ug = __builtin_amdgcn_readfirstlane(ug);
+  const int q0 = cu_q[b], q1 = cu_q[b + 1];
+  int L = ap->seq_lens[b];
+  const int qlen = q1 - q0;
+  L = L < ap->max_seq ? L : ap->max_seq;
+  PrefillRange rg = prefill_range(qlen, L, G, ug);
+  rg.units = __builtin_amdgcn_readfirstlane(rg.units);
+  rg.kend = __builtin_amdgcn_readfirstlane(rg.kend);
+  rg.n_steps = __builtin_amdgcn_readfirstlane(rg.n_steps);
+  if (4 * ug < rg.units) {  // else no query: the whole workgroup goes on together
+  const int all_steps = rg.n_steps > 0 ? rg.n_steps : 1;  // as the shared line counts them
+  int take = all_steps - s_begin;
+  if constexpr (SHARED) {
+    take = steps_left < take ? static_cast<int>(steps_left) : take;
+    __syncthreads();  // the LDS of the unit group before (or of the prefix) is free
+  }
+  const bool partial = SHARED && take < all_steps;
+  const bool active = 4 * ug + wave < rg.units;  // an idle wave still copies its tile of every step
+  const int unit = active ? 4 * ug + wave : rg.units - 1;
+  const int qt = __builtin_amdgcn_readfirstlane(unit / G);
   const int t0 = qt * 32;
-  if (t0 >= qlen) return;  // the whole workgroup leaves together
-  const int h_local = hg * kPrefillWaves + wave;
-  const bool active = h_local < G;  // an idle wave still copies its tile of every step
-  const int h = kvh * G + (active ? h_local : 0);
+  const int h = kvh * G.d + (unit - qt * G.d);
   const int ctx = L - qlen;
-  // this lane's output row (query t0 + l % 32), formed before the key loop
-  uint16_t *const op = out + static_cast<int64_t>(q0 + t0 + n) * o_st + static_cast<int64_t>(h) * o_sh;
-
   // Q^T operand j: lane l holds d = 16 j + 8 (l/32) .. + 7 of query t0 + l % 32.
   bf16x8 qb[D / 16];
   {
     const int tok = t0 + n;
     const bool valid = active && tok < qlen;
-    const uint16_t *qp = q + static_cast<int64_t>(q0 + (tok < qlen ? tok : t0)) * q_st + static_cast<int64_t>(h) * q_sh;
+    const uint16_t *qp =
+        ap->q + static_cast<int64_t>(q0 + (tok < qlen ? tok : t0)) * ap->q_st + static_cast<int64_t>(h) * ap->q_sh;
 #pragma unroll
     for (int j = 0; j < D / 16; ++j) {
       u32x4 w = *reinterpret_cast<const u32x4 *>(qp + 16 * j + 8 * hh);
@@ -156,12 +382,13 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(
     for (int r = 0; r < 16; ++r) o[c][r] = 0.f;
   float m_ref = -INFINITY, l_part = 0.f;
 
-  const int last = (t0 + 32 < qlen ? t0 + 32 : qlen) - 1;
-  const int kend = ctx + last + 1;  // keys [0, kend)
-  const int n_tiles = kend > 0 ? (kend + 15) / 16 : 0;
-  const int n_steps = (n_tiles + 3) / 4;
+  // The steps taken here; key and query positions from here on count from their first key.
+  const int key0 = 64 * s_begin;
+  const int kend = rg.kend - key0;
+  const int n_steps = rg.n_steps - s_begin < take ? rg.n_steps - s_begin : take;
+  const int n_tiles = (kend + 15) / 16 < 4 * n_steps ? (kend + 15) / 16 : 4 * n_steps;
   const int region = D * BS * ESZ;
-  const int min_pos = ctx + t0;  // the smallest query position of the workgroup
+  const int min_pos = ctx + t0 - key0;  // the smallest query position of the wave
 
   // Copy k of lane l moves piece p = 64 k + l of the wave's tile's K or V
   // (LDS offset 16 p). K piece p (both dtypes: 16-byte chunks): chunk p >> 4,
@@ -176,12 +403,13 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(
   const uint32_t ldsk0 = lds_addr(ldsk), ldsv0 = lds_addr(ldsv);
   const uint32_t stgk0 = lds_addr(stgk), stgv0 = lds_addr(stgv);
   float ks_next = 1.f, vs_next = 1.f, vs_stage = 1.f;  // fp8 scales: last K issued, its V, the staged V
-  const int32_t *btrow = bt + b * bt_stride;
-  int bix = (16 * wave) / BS;
-  int o0 = 16 * wave - bix * BS;
-  const int dbix = 64 / BS, do0 = 64 - dbix * BS;
-  int wbase = 0;  // the window: lane i holds the id of block wbase + i
-  int win = load_i32_drained(btrow, lane, Mb);
+  const int32_t *btrow = ap->bt + b * ap->bt_stride;
+  const FastDiv by_BS = ap->by_BS;
+  int bix = (key0 + 16 * wave) / by_BS;
+  int o0 = key0 + 16 * wave - bix * BS;
+  const int dbix = 64 / by_BS, do0 = 64 - dbix * BS;
+  int wbase = bix;  // the window: lane i holds the id of block wbase + i
+  int win = load_i32_drained(btrow, wbase + lane, Mb);
   int64_t vbase = 0;  // V of the wave's tile of the step whose K went out last: cache offset
   auto has_tile = [&](int s) { return s < n_steps && 4 * s + wave < n_tiles; };  // uniform
   // K of the wave's tile of step s into K slot `slot` (fp8: into the staging area)
@@ -477,8 +705,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(
     {
       qk(0, a0, a1);
       mask(0, a0, a1);
-      // the reference maximum starts at the first step's row maximum (every
-      // query sees key 0, so it is finite)
+      // the reference maximum starts at the first step's row maximum (a query
+      // that sees no key of it -- only past the unit group's first -- sees none at all)
       float mt = fmaxf(a0[0], a1[0]);
 #pragma unroll
       for (int r = 1; r < 16; ++r) mt = fmaxf(mt, fmaxf(a0[r], a1[r]));
@@ -508,26 +736,207 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(
       tail(s, a0, a1);
     }
   }
-  const int tok = t0 + n;
-  if (!active || tok >= qlen) return;
+  if (active) {
+  const PrefillArgs *ae = &kernel_args;  // SHARED: the epilogue's arguments are not held through the key loop
+  if constexpr (SHARED) ae = &prefill_args();
   float l = l_part;
   {
     const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(x[0]) + __uint_as_float(x[1]);
   }
-  // An attention sink (a zero-value logit of head h, natural-log units) adds
-  // its weight against the row's reference maximum to the denominator.
-  if (sinks != nullptr) l += exp2f(sinks[h] * 1.4426950408889634f - m_ref);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (partial) {  // uniform
+    const int w = (id & 7) * (ae->pg.W / 8) + id / 8;
+    float *pp = ae->part + ((2 * static_cast<int64_t>(w) + (seg > 0 ? 1 : 0)) * 4 + wave) * prefill_part_floats<D>();
 #pragma unroll
-  for (int c = 0; c < D / 32; ++c) {
+    for (int c = 0; c < D / 32; ++c)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {  // d = 32 c + 8 g + 4 hh + 0..3
-      const u32x2 w = {pack_bf16x2(o[c][4 * g] * inv, o[c][4 * g + 1] * inv),
-                       pack_bf16x2(o[c][4 * g + 2] * inv, o[c][4 * g + 3] * inv)};
-      *reinterpret_cast<u32x2 *>(op + 32 * c + 8 * g + 4 * hh) = w;
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<floatx4 *>(pp + ((4 * c + g) * 64 + lane) * 4) =
+            floatx4{o[c][4 * g], o[c][4 * g + 1], o[c][4 * g + 2], o[c][4 * g + 3]};
+    // a query that saw no key of this part must not set the merged maximum
+    if (hh == 0) {
+      pp[32 * D + n] = l > 0.f ? m_ref : -INFINITY;
+      pp[32 * D + 32 + n] = l;
+    }
+  } else if (t0 + n < qlen) {
+    // An attention sink (a zero-value logit of head h, natural-log units) adds
+    // its weight against the row's reference maximum to the denominator.
+    if (ae->sinks != nullptr) l += exp2f(ae->sinks[h] * 1.4426950408889634f - m_ref);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    uint16_t *const op = ae->out + static_cast<int64_t>(q0 + t0 + n) * ae->o_st + static_cast<int64_t>(h) * ae->o_sh;
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {  // d = 32 c + 8 g + 4 hh + 0..3
+        const u32x2 w = {pack_bf16x2(o[c][4 * g] * inv, o[c][4 * g + 1] * inv),
+                         pack_bf16x2(o[c][4 * g + 2] * inv, o[c][4 * g + 3] * inv)};
+        *reinterpret_cast<u32x2 *>(op + 32 * c + 8 * g + 4 * hh) = w;
+      }
     }
   }
+  }
+  if constexpr (SHARED) {
+    steps_left -= take;
+    ++seg;
+  }
+  }
+  if constexpr (!SHARED) break;
+  if (steps_left <= 0) break;
+  s_begin = 0;
+  const PrefillArgs &an = prefill_args();
+  if (++ug == an.pg.n_ug) {
+    ug = 0;
+    if (++b == an.pg.batch) {
+      b = 0;
+      if (++kvh == an.Hkv) break;  // never with steps left
+    }
+  }
+  }
+}
+
+// Log-sum-exp merge of a shared launch's partials: one wave per unit and 32
+// output columns (blockIdx.y), in the lanes' accumulator layout of the
+// attention kernel; a unit group that one workgroup took whole was finished
+// there. Bound by reading the partials (66 KB per part at d=128).
+template <int D>
+__global__ __launch_bounds__(64 * kPrefillWaves) void prefill_merge_kernel(
+    const float *__restrict__ part, uint16_t *__restrict__ out, int64_t o_st, int64_t o_sh,
+    const int32_t *__restrict__ cu_q, const int32_t *__restrict__ seq_lens, int max_seq, int Hkv, PrefillGrid pg,
+    const float *__restrict__ sinks) {
+  constexpr int PF = prefill_part_floats<D>();
+  __shared__ int pfx[kPrefillEntries + 1];
+  __shared__ int red[kPrefillWaves];
+  const int total = prefill_prefix(pfx, red, cu_q, seq_lens, max_seq, pg);
+  const int E = pg.batch * pg.n_ug;
+  const int kvh = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x / E));
+  const int e = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x - kvh * E));
+  const int c = blockIdx.y;
+  const int b = __builtin_amdgcn_readfirstlane(e / pg.by_ug);
+  const int ug = e - b * pg.n_ug;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63, n = lane & 31, hh = lane >> 5;
+  const int q0 = cu_q[b];
+  const int qlen = cu_q[b + 1] - q0;
+  const FastDiv G = pg.by_G;
+  const int units = qlen > 0 ? ((qlen + 31) >> 5) * G.d : 0;
+  const int unit = 4 * ug + wave;
+  const int n_e = __builtin_amdgcn_readfirstlane(pfx[e + 1] - pfx[e]);
+  if (n_e <= 0 || unit >= units) return;
+  // The workgroups whose shares [share(w), share(w + 1)) meet this group's steps [x0, x0 + n_e).
+  const int64_t T = static_cast<int64_t>(total) * Hkv;
+  const int W = T < pg.W ? static_cast<int>(T) : pg.W;
+  const int64_t x0 = static_cast<int64_t>(kvh) * total + __builtin_amdgcn_readfirstlane(pfx[e]);
+  const int64_t x1 = x0 + n_e;
+  int w0 = static_cast<int>(x0 * W / T);
+  while (prefill_share(w0 + 1, T, W) <= x0) ++w0;
+  while (prefill_share(w0, T, W) > x0) --w0;
+  int w1 = w0;  // last
+  while (prefill_share(w1 + 1, T, W) < x1) ++w1;
+  w0 = __builtin_amdgcn_readfirstlane(w0);
+  w1 = __builtin_amdgcn_readfirstlane(w1);
+  if (w0 == w1) return;
+  // The group is its workgroup's first unit group iff the share starts inside it (or with it).
+  const float *p0 = part + ((2 * static_cast<int64_t>(w0) + (prefill_share(w0, T, W) < x0 ? 1 : 0)) * 4 + wave) * PF;
+  const float *pn = part + (2 * static_cast<int64_t>(w0 + 1) * 4 + wave) * PF;  // the later parts, 8 PF apart
+  const int np = w1 - w0;
+  const int qt = __builtin_amdgcn_readfirstlane(unit / G);
+  const int h = kvh * G.d + (unit - qt * G.d);
+  float M = p0[32 * D + n];
+#pragma unroll 4
+  for (int s = 0; s < np; ++s) M = fmaxf(M, pn[s * (8 * PF) + 32 * D + n]);
+  const float m_use = M == -INFINITY ? 0.f : M;
+  float l = 0.f;
+  floatx4 acc[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) acc[g] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto add = [&](const float *ps) {
+    const float w = exp2f(ps[32 * D + n] - m_use);
+    l += w * ps[32 * D + 32 + n];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const floatx4 x = *reinterpret_cast<const floatx4 *>(ps + ((4 * c + g) * 64 + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[g][i] += w * x[i];
+    }
+  };
+  add(p0);
+#pragma unroll 4
+  for (int s = 0; s < np; ++s) add(pn + s * (8 * PF));
+  const int tok = 32 * qt + n;
+  if (tok >= qlen) return;
+  if (sinks != nullptr) l += exp2f(sinks[h] * 1.4426950408889634f - m_use);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t *op = out + static_cast<int64_t>(q0 + tok) * o_st + static_cast<int64_t>(h) * o_sh;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const u32x2 w = {pack_bf16x2(acc[g][0] * inv, acc[g][1] * inv), pack_bf16x2(acc[g][2] * inv, acc[g][3] * inv)};
+    *reinterpret_cast<u32x2 *>(op + 32 * c + 8 * g + 4 * hh) = w;
+  }
+}
+
+// The launch's grid. With a workspace (may_share), the steps are shared over
+// W workgroups where that is expected to be faster; share > 0 sets W.
+static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int max_query_len, int max_seq,
+                                int share, bool may_share) {
+  PrefillGrid pg;
+  const int64_t n_qt = (static_cast<int64_t>(max_query_len) + 31) / 32;
+  pg.n_ug = static_cast<int>((n_qt * G + 3) / 4);
+  pg.batch = batch;
+  const int64_t items = static_cast<int64_t>(batch) * Hkv;
+  const int64_t wgs = items * pg.n_ug;
+  pg.W = 0;
+  if (may_share && static_cast<int64_t>(batch) * pg.n_ug <= kPrefillEntries) {
+    if (share > 0) {
+      pg.W = (share + 7) / 8 * 8;
+    } else if (wgs < 4 * kPrefillCus && max_seq > kShareMinKeys) {
+      // Measured (us, plain -> shared): 4 x 37-250 new tokens over 5-15K keys at
+      // 28/4 heads 241 -> 131 (fp8 352 -> 131), 64 over 2K at 32/8 38 -> 23,
+      // 8 x 20-60 over 4-12K at 32/4 fp8 275 -> 82, 1,000 over 8K at 16/8 147 ->
+      // 87; but 16 x 16 over 1K 22.5 -> 27.3, one prompt of 1,500 tokens 36 -> 55
+      // and of 512 15 -> 29: short chains gain less than the partials and the
+      // second launch cost.
+      const double steps = max_seq > 64 ? max_seq / 64.0 : 1.0;
+      const double qsteps = max_query_len < max_seq ? max_query_len / 64.0 : steps;
+      // the host knows the longest lengths only: several sequences are taken
+      // to bring 0.6 of the longest one's work on average
+      const double T = wgs * (steps - 0.5 * qsteps) * (batch > 1 ? 0.6 : 1.0);
+      // plain: the longest chain or the chip's throughput, and a tail
+      const double alone = fp8 ? kStepFp8Us : kStepUs;
+      const double full = T / (2 * kPrefillCus) * kStepPairUs;
+      double best = fmax(steps * alone, full) + (wgs > kPrefillCus ? 0.3 * steps * alone : 0.0) + kLaunchUs;
+      best *= 0.75;  // shared only for a clear gain
+      for (int W = 64; W <= 2 * kPrefillCus; W += 64) {
+        const bool pair = W > kPrefillCus;
+        const double ts = T / W * (pair ? kStepPairUs : alone) + kPartUs * W * D / 128 +
+                          (pair ? 0.5 : 1.0) * kGroupUs * (1.0 + static_cast<double>(wgs) / W) + kShareUs;
+        if (ts < best) {
+          best = ts;
+          pg.W = W;
+        }
+      }
+    }
+  }
+  // Items are dealt to the eight XCDs in turn: R makes the KV heads of one
+  // sequence (its unit groups dealt over R XCDs where there are fewer than
+  // eight) cover all of them, so that sequences of different lengths load the
+  // XCDs alike (8 prompts of 438-1,314 tokens at 28/4 heads: 98 us so, 107
+  // with two sequences at a time on four XCDs each).
+  pg.R = 1;
+  while (static_cast<int64_t>(Hkv) * pg.R % 8 != 0) pg.R *= 2;
+  while (pg.R > 1 && pg.R > pg.n_ug) pg.R /= 2;
+  pg.n_inner = (pg.n_ug + pg.R - 1) / pg.R;
+  pg.n_sub = static_cast<int>(items * pg.R);
+  pg.log2R = 0;
+  while ((1 << pg.log2R) < pg.R) ++pg.log2R;
+  pg.by_G = fast_div(G);
+  pg.by_ug = fast_div(pg.n_ug);
+  pg.by_inner = fast_div(pg.n_inner);
+  pg.by_Hkv = fast_div(Hkv);
+  return pg;
+}
+
+static int64_t prefill_workspace(const PrefillGrid &pg, int D) {
+  return static_cast<int64_t>(pg.W) * 2 * 4 * (32 * D + 64) * 4;
 }
 
 }  // namespace wkv
@@ -540,8 +949,8 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
                           int64_t q_stride_h, void *out, int64_t out_stride_t, int64_t out_stride_h,
                           int32_t num_q_heads, const int32_t *cu_seqlens_q, const int32_t *seq_lens,
                           const int32_t *block_table, int64_t bt_stride, int32_t max_blocks_per_seq, int32_t batch,
-                          int32_t max_query_len, int32_t max_seq_len, float scale, const float *sinks,
-                          void *stream) {
+                          int32_t max_query_len, int32_t max_seq_len, float scale, int32_t workgroups,
+                          void *workspace, int64_t workspace_bytes, const float *sinks, void *stream) {
   int rc = check_cache(cache, -1);
   if (rc) return rc;
   WKV_CHECK_ARG(batch >= 0 && batch <= 65535, "batch must be in [0, 65535] (got %d)", batch);
@@ -574,12 +983,15 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
   WKV_CHECK_ARG(max_query_len > 0 && max_seq_len >= 0, "max_query_len must be > 0 and max_seq_len >= 0");
   WKV_CHECK_ARG(std::isfinite(scale), "scale must be finite");
   const int max_seq = max_seq_len < max_blocks_per_seq * BS ? max_seq_len : max_blocks_per_seq * BS;
+  WKV_CHECK_ARG(workgroups >= 0 && workgroups <= 65536, "workgroups must be in [0, 65536]");
+  WKV_CHECK_ARG(static_cast<int64_t>(batch) * Hkv <= INT32_MAX / 8, "batch * num_kv_heads too large");
   const bool fp8 = cache->kv_dtype == WKV_KV_FP8_E4M3;
-  const int n_hg = (G + kPrefillWaves - 1) / kPrefillWaves;
-  const int q_tile = 32;
-  const int n_qt = (max_query_len + q_tile - 1) / q_tile;
-  const int64_t n_items = static_cast<int64_t>(batch) * Hkv * n_hg;
-  const int64_t n_wg = (n_items + 7) / 8 * 8 * n_qt;
+  const PrefillGrid pg = prefill_grid(batch, Hkv, G, D, fp8, max_query_len, max_seq, workgroups, workspace != nullptr);
+  const int64_t need = prefill_workspace(pg, D);
+  if (need > 0)
+    WKV_CHECK_ARG(aligned16(workspace) && workspace_bytes >= need, "workspace too small: need %lld bytes, got %lld",
+                  (long long)need, (long long)workspace_bytes);
+  const int64_t n_wg = pg.W > 0 ? pg.W : (static_cast<int64_t>(pg.n_sub) + 7) / 8 * 8 * pg.n_inner;
   WKV_CHECK_ARG(n_wg <= INT32_MAX, "prefill grid too large");
   const dim3 grid(static_cast<unsigned>(n_wg));
   auto s = static_cast<hipStream_t>(stream);
@@ -588,18 +1000,38 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
   auto qq = static_cast<const uint16_t *>(q);
   auto oo = static_cast<uint16_t *>(out);
   const float scale_log2 = scale * 1.4426950408889634f;
-#define WKV_PREFILL(Dv, F8)                                                                                       \
-  prefill_gqa_kernel<Dv, F8><<<grid, 64 * kPrefillWaves, 0, s>>>(                                                \
-      kc, vc, cache->k_scale, cache->v_scale, qq, q_stride_t, q_stride_h, oo, out_stride_t, out_stride_h,       \
-      cu_seqlens_q, seq_lens, block_table, bt_stride, max_blocks_per_seq, max_seq, Hkv, G, n_hg, BS,           \
-      static_cast<int>(cache->num_blocks), scale_log2, n_qt, static_cast<int>(n_items), sinks)
+  const PrefillArgs args{kc, vc, cache->k_scale, cache->v_scale, qq, q_stride_t, q_stride_h, oo, out_stride_t,
+                         out_stride_h, cu_seqlens_q, seq_lens, block_table, bt_stride, max_blocks_per_seq, max_seq,
+                         Hkv, BS, static_cast<int>(cache->num_blocks), scale_log2, fast_div(BS), pg,
+                         static_cast<float *>(workspace), sinks};
+#define WKV_PREFILL_S(Dv, F8, SH) prefill_gqa_kernel<Dv, F8, SH><<<grid, 64 * kPrefillWaves, 0, s>>>(args)
+#define WKV_PREFILL(Dv, F8)         \
+  do {                              \
+    if (pg.W > 0)                   \
+      WKV_PREFILL_S(Dv, F8, true);  \
+    else                            \
+      WKV_PREFILL_S(Dv, F8, false); \
+  } while (0)
   if (D == 128) {
     if (fp8) WKV_PREFILL(128, true); else WKV_PREFILL(128, false);
   } else {
     if (fp8) WKV_PREFILL(64, true); else WKV_PREFILL(64, false);
   }
 #undef WKV_PREFILL
+#undef WKV_PREFILL_S
   WKV_CHECK_LAUNCH("paged prefill");
+  if (pg.W > 0) {
+    const dim3 mgrid(static_cast<unsigned>(Hkv * batch * pg.n_ug), static_cast<unsigned>(D / 32));
+    if (D == 128)
+      prefill_merge_kernel<128><<<mgrid, 64 * kPrefillWaves, 0, s>>>(static_cast<const float *>(workspace), oo,
+                                                                     out_stride_t, out_stride_h, cu_seqlens_q, seq_lens,
+                                                                     max_seq, Hkv, pg, sinks);
+    else
+      prefill_merge_kernel<64><<<mgrid, 64 * kPrefillWaves, 0, s>>>(static_cast<const float *>(workspace), oo,
+                                                                    out_stride_t, out_stride_h, cu_seqlens_q, seq_lens,
+                                                                    max_seq, Hkv, pg, sinks);
+    WKV_CHECK_LAUNCH("paged prefill merge");
+  }
   return WKV_OK;
 }
 
@@ -613,7 +1045,7 @@ extern "C" int wkv_prefill_gqa(const wkv_cache_t *cache, const void *key, int64_
   return launch_prefill(cache, key, key_stride_t, key_stride_h, value, value_stride_t, value_stride_h, slot_mapping,
                         num_tokens, q, q_stride_t, q_stride_h, out, out_stride_t, out_stride_h, num_q_heads,
                         cu_seqlens_q, seq_lens, block_table, bt_stride, max_blocks_per_seq, batch, max_query_len,
-                        max_seq_len, scale, nullptr, stream);
+                        max_seq_len, scale, 0, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int wkv_prefill_gqa_sinks(const wkv_cache_t *cache, const void *key, int64_t key_stride_t,
@@ -629,5 +1061,34 @@ extern "C" int wkv_prefill_gqa_sinks(const wkv_cache_t *cache, const void *key, 
   return launch_prefill(cache, key, key_stride_t, key_stride_h, value, value_stride_t, value_stride_h, slot_mapping,
                         num_tokens, q, q_stride_t, q_stride_h, out, out_stride_t, out_stride_h, num_q_heads,
                         cu_seqlens_q, seq_lens, block_table, bt_stride, max_blocks_per_seq, batch, max_query_len,
-                        max_seq_len, scale, sinks, stream);
+                        max_seq_len, scale, 0, nullptr, 0, sinks, stream);
+}
+
+extern "C" int64_t wkv_prefill_workspace_size(int32_t batch, int32_t kv_dtype, int32_t num_kv_heads,
+                                              int32_t num_q_heads, int32_t head_dim, int32_t max_query_len,
+                                              int32_t max_seq_len, int32_t workgroups) {
+  if (batch < 0 || batch > 65535 || num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
+      head_dim <= 0 || max_query_len < 0 || max_seq_len < 0 || workgroups < 0 || workgroups > 65536)
+    return -1;
+  if (batch == 0 || max_query_len == 0 || static_cast<int64_t>(batch) * num_kv_heads > INT32_MAX / 8) return 0;
+  return prefill_workspace(prefill_grid(batch, num_kv_heads, num_q_heads / num_kv_heads, head_dim,
+                                        kv_dtype == WKV_KV_FP8_E4M3, max_query_len, max_seq_len, workgroups, true),
+                           head_dim);
+}
+
+extern "C" int wkv_prefill_gqa_shared(const wkv_cache_t *cache, const void *key, int64_t key_stride_t,
+                                     int64_t key_stride_h, const void *value, int64_t value_stride_t,
+                                     int64_t value_stride_h, const int64_t *slot_mapping, int64_t num_tokens,
+                                     const void *q, int64_t q_stride_t, int64_t q_stride_h, void *out,
+                                     int64_t out_stride_t, int64_t out_stride_h, int32_t num_q_heads,
+                                     const int32_t *cu_seqlens_q, const int32_t *seq_lens,
+                                     const int32_t *block_table, int64_t bt_stride, int32_t max_blocks_per_seq,
+                                     int32_t batch, int32_t max_query_len, int32_t max_seq_len, float scale,
+                                     int32_t workgroups, void *workspace, int64_t workspace_bytes,
+                                     const float *sinks, void *stream) {
+  WKV_CHECK_ARG(reinterpret_cast<uintptr_t>(sinks) % 4 == 0, "sinks must be fp32");
+  return launch_prefill(cache, key, key_stride_t, key_stride_h, value, value_stride_t, value_stride_h, slot_mapping,
+                        num_tokens, q, q_stride_t, q_stride_h, out, out_stride_t, out_stride_h, num_q_heads,
+                        cu_seqlens_q, seq_lens, block_table, bt_stride, max_blocks_per_seq, batch, max_query_len,
+                        max_seq_len, scale, workgroups, workspace, workspace_bytes, sinks, stream);
 }

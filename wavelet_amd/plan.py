@@ -23,7 +23,7 @@ import torch
 
 from . import _lib
 from .attention import _workspace, decode_plan
-from .cache import PagedKVCache, _require_cuda, check_tables
+from .cache import KV_DTYPES, PagedKVCache, _require_cuda, check_tables
 
 
 # Smallest B * Hkv * max_seq_len (token-heads) for which DecodeStep orders
@@ -411,6 +411,13 @@ class PrefillStep:
         T = slot_mapping.numel()
         self.lib = lib = _lib.load()
         self.stream = torch.cuda.current_stream(dev).cuda_stream
+        c0 = caches[0]
+        need = max(lib.wkv_prefill_workspace_size(
+            batch, KV_DTYPES[c.kv_dtype], c.num_kv_heads, qq.shape[1], c.head_dim, int(max_query_len),
+            min(int(max_seq_len), self.block_table.shape[1] * c0.block_size), 0) for c, qq in zip(caches, q))
+        # the plan's own scratch for a small grid's shared key ranges (None: nothing is shared)
+        self.workspace = torch.empty(need, dtype=torch.uint8, device=dev) if need > 0 else None
+        split = (0, self.workspace.data_ptr(), need, None) if need > 0 else (0, None, 0, None)
         self.calls = []
         for layer, cache in enumerate(caches):
             qq, kk, vv, oo = q[layer], key[layer], value[layer], out[layer]
@@ -426,7 +433,7 @@ class PrefillStep:
             tail = (qq.data_ptr(), qq.stride(0), qq.stride(1), oo.data_ptr(), oo.stride(0), oo.stride(1), hq,
                     cu_seqlens_q.data_ptr(), self.seq_lens.data_ptr(), self.block_table.data_ptr(),
                     self.block_table.stride(0), self.block_table.shape[1], batch, int(max_query_len),
-                    int(max_seq_len), ctypes.c_float(scale), self.stream)
+                    int(max_seq_len), ctypes.c_float(scale), *split, self.stream)
             fn = lib.wkv_append_fp8 if cache.kv_dtype == "fp8_e4m3" else lib.wkv_append
             self.calls.append((fn, (desc, *kv, T, self.stream), (desc, *kv, T, *tail),
                                (desc, None, 0, 0, None, 0, 0, None, 0, *tail)))
@@ -441,14 +448,14 @@ class PrefillStep:
 
     def attend(self, layer: int) -> None:
         self._live.check(layer)
-        rc = self.lib.wkv_prefill_gqa(*self.calls[layer][3])
+        rc = self.lib.wkv_prefill_gqa_shared(*self.calls[layer][3])
         if rc:
             _lib.check(rc, f"prefill layer {layer}")
 
     def step_layer(self, layer: int) -> None:
         """Append + causal attention of one layer (two launches: the append, then the attention)."""
         self._live.check(layer)
-        rc = self.lib.wkv_prefill_gqa(*self.calls[layer][2])
+        rc = self.lib.wkv_prefill_gqa_shared(*self.calls[layer][2])
         if rc:
             _lib.check(rc, f"append+prefill layer {layer}")
 
