@@ -401,6 +401,21 @@ int wkv_sample(const void *logits, int32_t logits_dtype, int64_t row_stride, int
                const float *repetition_penalty, const uint32_t *seen_tokens, const uint64_t *seeds, int64_t step,
                int64_t *out_tokens, float *out_logprobs, uint32_t *out_mask, int32_t *out_counts, void *stream);
 
+/* wkv_sample with a workspace, so that a call over few rows drawn from the
+ * whole vocabulary (top_k, top_p and min_p all NULL) can cut each row into
+ * slices that share the chip (three launches instead of one). The same
+ * arguments and results as wkv_sample: tokens, masks and counts are identical,
+ * a logprob may differ in the last bits where the kept mass is a float sum.
+ * workspace: wkv_sample_workspace_size() bytes of scratch, 16-byte aligned (0 =
+ * rows are never cut at this size; workspace may then be NULL). */
+int64_t wkv_sample_workspace_size(int32_t batch, int32_t vocab);
+
+int wkv_sample_sliced(const void *logits, int32_t logits_dtype, int64_t row_stride, int32_t batch, int32_t vocab,
+                      const float *temperature, const int32_t *top_k, const float *top_p, const float *min_p,
+                      const float *repetition_penalty, const uint32_t *seen_tokens, const uint64_t *seeds,
+                      int64_t step, int64_t *out_tokens, float *out_logprobs, uint32_t *out_mask,
+                      int32_t *out_counts, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* Weight-absorbed MLA decode over the latent cache:
  *   s = (q_nope . c_kv + q_pe . k_pe) * scale; o = softmax(s) . c_kv
  * q_nope [batch, num_heads, kv_lora_rank], q_pe [batch, num_heads, rope_dim]

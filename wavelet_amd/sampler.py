@@ -19,6 +19,8 @@ from . import _lib
 from .cache import _require_cuda, _stream
 
 
+_SLICE_MIN_VOCAB = 40960  # the library cuts no row of fewer logits
+
 # Ranges a scalar parameter must lie in (the reference's sampling config:
 # configs/config.py:854-859); per-row tensors are not read back (that would
 # synchronise): the kernel keeps at least the row's maximum whatever min_p is.
@@ -127,10 +129,20 @@ def sample(
     def ptr(x):
         return None if x is None else x.data_ptr()
 
-    rc = _lib.load().wkv_sample(
-        logits.data_ptr(), 0 if logits.dtype == torch.float32 else 1, logits.stride(0), batch, vocab, ptr(t), ptr(k),
-        ptr(p), ptr(mp), ptr(rp), ptr(seen), ptr(seeds), int(step), tokens.data_ptr(), logprobs.data_ptr(),
-        ptr(mask), ptr(counts), _stream(dev))
+    lib = _lib.load()
+    args = (logits.data_ptr(), 0 if logits.dtype == torch.float32 else 1, logits.stride(0), batch, vocab, ptr(t),
+            ptr(k), ptr(p), ptr(mp), ptr(rp), ptr(seen), ptr(seeds), int(step), tokens.data_ptr(),
+            logprobs.data_ptr(), ptr(mask), ptr(counts))
+    # few rows drawn from the whole vocabulary are cut into slices, through scratch from the
+    # caching allocator on the call's own stream
+    need = 0
+    if vocab > _SLICE_MIN_VOCAB and k is None and p is None and mp is None:
+        need = lib.wkv_sample_workspace_size(batch, vocab)
+    if need > 0:
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        rc = lib.wkv_sample_sliced(*args, ws.data_ptr(), need, _stream(dev))
+    else:
+        rc = lib.wkv_sample(*args, _stream(dev))
     _lib.check(rc, "sample")
     return tokens, logprobs, mask, counts
 
