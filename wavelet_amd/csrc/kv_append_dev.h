@@ -19,6 +19,19 @@ __device__ __forceinline__ int64_t fp8_v_index(int64_t blk, int h, int H, int BS
   return ((blk * H + h) * D + d) * BS + off;
 }
 
+// Four e4m3 codes times `ratio`, a power of two below 1, by the hardware
+// conversions: code by code e4m3_encode(e4m3_decode(c) * ratio) (the products
+// are bf16 values, for which the two encoders agree bit for bit). NaN codes
+// are kept as they are, as the encoder keeps them.
+__device__ __forceinline__ uint32_t fp8x4_rescale(uint32_t c, float ratio) {
+  const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(c), false);
+  const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(c), true);
+  int r = __builtin_amdgcn_cvt_pk_fp8_f32(lo[0] * ratio, lo[1] * ratio, 0, false);
+  r = __builtin_amdgcn_cvt_pk_fp8_f32(hi[0] * ratio, hi[1] * ratio, r, true);
+  const uint32_t nan = ((((c & 0x7f7f7f7fu) + 0x01010101u) & 0x80808080u) >> 7) * 0xffu;  // bytes of code 0x7f or 0xff
+  return (static_cast<uint32_t>(r) & ~nan) | (c & nan);
+}
+
 // Re-encodes the codes at offsets [0, first) of the (blk, h) region of K (IS_V
 // false) or V at a grown scale: each code times `ratio`, an exact power of two
 // below 1 (e4m3_encode(e4m3_decode(c) * ratio), code by code, as the oracle
@@ -49,15 +62,10 @@ __device__ __forceinline__ void fp8_reencode_block(uint8_t *__restrict__ cache, 
       u32x4 o = w[k];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int tok = IS_V ? tok0 + 4 * j + b : tok0;
-          if (tok < first) {
-            const uint32_t c = (o[j] >> (8 * b)) & 0xffu;
-            const uint32_t n = e4m3_encode(e4m3_decode(c) * ratio);
-            o[j] = (o[j] & ~(0xffu << (8 * b))) | (n << (8 * b));
-          }
-        }
+        // the bytes of this word before `first`: all of them (K: a piece is one token)
+        const int n = IS_V ? first - (tok0 + 4 * j) : 4;
+        const uint32_t m = n >= 4 ? 0xffffffffu : (n <= 0 ? 0u : (1u << (8 * n)) - 1u);
+        o[j] = (o[j] & ~m) | (fp8x4_rescale(o[j], ratio) & m);
       }
       base[p] = o;
     }
@@ -232,69 +240,6 @@ __device__ __forceinline__ void fp8_append_token_kv(uint8_t *__restrict__ kc, ui
   }
 }
 
-// The same append with 16-byte source loads and 16-byte K stores, and the
-// quantisation as a product with 1 / scale (a power of two: x * (1 / s) and
-// x / s round the same exact value, so the codes are identical). The source
-// rows must be 16-byte aligned (the host checks). K: a lane quantises one
-// (token, 16-d chunk) piece into 16 contiguous code bytes; V: one d row's
-// byte per token, as before.
-template <int D, bool IS_V>
-__device__ void fp8_append_run_vec(uint8_t *__restrict__ cache, float *__restrict__ scales,
-                                   const uint16_t *__restrict__ src, int64_t st, int64_t sh,
-                                   const int64_t *__restrict__ slots, int64_t t, int r, int64_t blk, int first, int h,
-                                   int H, int BS) {
-  const int lane = threadIdx.x & 63;
-  float amax = 0.0f;
-  for (int e = lane; e < r * (D / 8); e += 64) {
-    const int tok = e / (D / 8), g = e % (D / 8);
-    const u32x4 w = *reinterpret_cast<const u32x4 *>(src + (t + tok) * st + h * sh + 8 * g);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      amax = fmaxf(amax, fmaxf(fabsf(__uint_as_float(w[j] << 16)), fabsf(__uint_as_float(w[j] & 0xffff0000u))));
-  }
-  amax = wave_max(amax);
-  const float s_new = pow2_scale(amax);
-  float s = s_new;
-  if (first != 0) {
-    const float s_old = scales[blk * H + h];
-    s = (s_new > s_old) ? s_new : s_old;
-    if (s > s_old) {  // the block's earlier codes are re-encoded at the grown scale
-      fp8_reencode_block<D, IS_V>(cache, blk, h, H, BS, first, s_old / s);  // exact power-of-two ratio
-    }
-  }
-  const float inv = 1.0f / s;  // exact: s is a power of two in [2^-42, 2^119]
-  auto q = [&](float x) {
-    float v = x * inv;
-    v = (v != v) ? v : fminf(fmaxf(v, -448.0f), 448.0f);
-    return e4m3_encode(v);
-  };
-  if constexpr (!IS_V) {
-    for (int e = lane; e < r * (D / 16); e += 64) {
-      const int tok = e / (D / 16), c = e % (D / 16);
-      const int off = static_cast<int>(slots[t + tok] % BS);
-      const uint16_t *p = src + (t + tok) * st + h * sh + 16 * c;
-      const u32x4 w0 = *reinterpret_cast<const u32x4 *>(p), w1 = *reinterpret_cast<const u32x4 *>(p + 8);
-      u32x4 out;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const u32x4 &w = j < 2 ? w0 : w1;
-        const uint32_t lo = w[(2 * j) & 3], hi = w[(2 * j + 1) & 3];
-        out[j] = q(__uint_as_float(lo << 16)) | (q(__uint_as_float(lo & 0xffff0000u)) << 8) |
-                 (q(__uint_as_float(hi << 16)) << 16) | (q(__uint_as_float(hi & 0xffff0000u)) << 24);
-      }
-      *reinterpret_cast<u32x4 *>(cache + fp8_k_index<D>(blk, h, H, BS, off, 16 * c)) = out;
-    }
-  } else {
-    for (int e = lane; e < r * D; e += 64) {
-      const int tok = e / D, d = e % D;
-      const int off = static_cast<int>(slots[t + tok] % BS);
-      const float x = bf16_bits_to_f32(src[(t + tok) * st + h * sh + d]);
-      cache[fp8_v_index<D>(blk, h, H, BS, off, d)] = static_cast<uint8_t>(q(x));
-    }
-  }
-  if (lane == 0) scales[blk * H + h] = s;
-}
-
 // Codes of a and b (after the clamp to +-448; never NaN here) in bytes
 // 2 w, 2 w + 1 of `old`, by the hardware conversion: for every finite input
 // bit-identical to e4m3_encode (checked on the GPU for all bf16 patterns at
@@ -316,11 +261,135 @@ __device__ __forceinline__ u32x2 e4m3_pack8(uint32_t w0, uint32_t w1, uint32_t w
   return r;
 }
 
+// fp8 append of one run (tokens t..t+r-1, all in block blk, the first at offset
+// `first`) for one head, K and V together, by one wave: the codes, scales and
+// re-encodes of fp8_append_one. Bound by memory round trips, so the run goes in
+// pieces of 16 tokens whose rows, slots and old scales are all requested before
+// the first is used (K: lane l holds token l % 16, 16-d chunks l / 16 + 4 j; V:
+// RV = D / 64 rows of every token), and a run of one piece -- any run of a
+// 16-token block -- stays in registers between its maximum and its codes; a
+// longer run reads its pieces twice. Loads of tokens past the run repeat its
+// last token (no effect on the maximum) and are not stored. 574 tokens in four
+// ragged runs over partly filled blocks, 4 heads: 22.7 us with K and V one
+// after the other and V a token at a time, 11.1 us so. Source rows 16-byte
+// aligned (the host checks).
+template <int D>
+__device__ void fp8_append_run_kv(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc, float *__restrict__ ks,
+                                  float *__restrict__ vs, const uint16_t *__restrict__ key, int64_t kst, int64_t ksh,
+                                  const uint16_t *__restrict__ val, int64_t vst, int64_t vsh,
+                                  const int64_t *__restrict__ slots, int64_t t, int r, int64_t blk, int first, int h,
+                                  int H, int BS) {
+  constexpr int P = 16, NC = D / 64, RV = D / 64;
+  const int lane = threadIdx.x & 63, m = lane & 15;
+  const int64_t si = blk * H + h;
+  const float sk_old = first != 0 ? ks[si] : 0.f, sv_old = first != 0 ? vs[si] : 0.f;
+  u32x4 kw[NC][2];
+  uint32_t vw[P];
+  int off = 0;  // offset in the block of the piece's token m
+  auto load = [&](int p0) __attribute__((always_inline)) {
+    const int last = (r - p0 < P ? r - p0 : P) - 1;
+    const int64_t tm = t + p0 + (m < last ? m : last);
+    off = static_cast<int>(slots[tm] - blk * BS);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const uint16_t *p = key + tm * kst + h * ksh + 16 * ((lane >> 4) + 4 * j);
+      kw[j][0] = *reinterpret_cast<const u32x4 *>(p);
+      kw[j][1] = *reinterpret_cast<const u32x4 *>(p + 8);
+    }
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const uint16_t *p = val + (t + p0 + (i < last ? i : last)) * vst + h * vsh + RV * lane;
+      if constexpr (RV == 2)
+        vw[i] = *reinterpret_cast<const uint32_t *>(p);
+      else
+        vw[i] = *p;
+    }
+  };
+  // Largest magnitude bits (as bf16); a NaN counts as none, as fmaxf has it, and is remembered.
+  uint32_t ka = 0u, va = 0u;
+  bool nan = false;
+  auto mag = [&](uint32_t a, uint32_t w) __attribute__((always_inline)) {
+    const uint32_t x = w & 0x7fffu, y = (w >> 16) & 0x7fffu;
+    nan = nan || x > 0x7f80u || y > 0x7f80u;
+    return max(a, max(x > 0x7f80u ? 0u : x, y > 0x7f80u ? 0u : y));
+  };
+  for (int p0 = 0; p0 < r; p0 += P) {  // uniform
+    load(p0);
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ka = mag(ka, kw[j][q][e]);
+#pragma unroll
+    for (int i = 0; i < P; ++i) va = mag(va, vw[i]);
+  }
+  ka = wave_reduce(ka, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+  va = wave_reduce(va, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+  const bool any_nan = __any(nan);
+  float sk = pow2_scale(__uint_as_float(ka << 16)), sv = pow2_scale(__uint_as_float(va << 16));
+  if (first != 0) {  // the block's earlier codes are re-encoded at a grown scale (exact power-of-two ratio)
+    if (sk > sk_old)
+      fp8_reencode_block<D, false>(kc, blk, h, H, BS, first, sk_old / sk);
+    else
+      sk = sk_old;
+    if (sv > sv_old)
+      fp8_reencode_block<D, true>(vc, blk, h, H, BS, first, sv_old / sv);
+    else
+      sv = sv_old;
+  }
+  // exact: powers of two in [2^-42, 2^119], so x * (1 / s) and x / s round the same value
+  const float ik = 1.0f / sk, iv = 1.0f / sv;
+  auto q = [](uint32_t bits, float inv) {  // a NaN's code as e4m3_encode has it
+    float v = __uint_as_float(bits << 16) * inv;
+    v = (v != v) ? v : fminf(fmaxf(v, -448.0f), 448.0f);
+    return e4m3_encode(v);
+  };
+  auto pack8 = [&](uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, float inv) __attribute__((always_inline)) {
+    if (!any_nan) return e4m3_pack8(w0, w1, w2, w3, inv);  // uniform
+    u32x2 o;
+    o[0] = q(w0 & 0xffffu, inv) | (q(w0 >> 16, inv) << 8) | (q(w1 & 0xffffu, inv) << 16) | (q(w1 >> 16, inv) << 24);
+    o[1] = q(w2 & 0xffffu, inv) | (q(w2 >> 16, inv) << 8) | (q(w3 & 0xffffu, inv) << 16) | (q(w3 >> 16, inv) << 24);
+    return o;
+  };
+  for (int p0 = 0; p0 < r; p0 += P) {
+    if (r > P) load(p0);
+    const int n = r - p0 < P ? r - p0 : P;
+    if (m < n) {
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        const u32x2 a = pack8(kw[j][0][0], kw[j][0][1], kw[j][0][2], kw[j][0][3], ik);
+        const u32x2 b = pack8(kw[j][1][0], kw[j][1][1], kw[j][1][2], kw[j][1][3], ik);
+        *reinterpret_cast<u32x4 *>(kc + fp8_k_index<D>(blk, h, H, BS, off, 16 * ((lane >> 4) + 4 * j))) =
+            u32x4{a[0], a[1], b[0], b[1]};
+      }
+    }
+#pragma unroll
+    for (int rr = 0; rr < RV; ++rr) {
+      // row RV lane + rr: the rr-th half of every token's word, a byte per token
+      uint8_t *row = vc + fp8_v_index<D>(blk, h, H, BS, 0, RV * lane + rr);
+      auto pair = [&](int i) { return ((vw[i] >> (16 * rr)) & 0xffffu) | (((vw[i + 1] >> (16 * rr)) & 0xffffu) << 16); };
+#pragma unroll
+      for (int g = 0; g < P; g += 8) {
+        if (g >= n) break;  // uniform
+        const u32x2 c = pack8(pair(g), pair(g + 2), pair(g + 4), pair(g + 6), iv);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (g + i < n) row[__builtin_amdgcn_readlane(off, g + i)] = static_cast<uint8_t>(c[i >> 2] >> (8 * (i & 3)));
+      }
+    }
+  }
+  if (lane == 0) {
+    ks[si] = sk;
+    vs[si] = sv;
+  }
+}
+
 // fp8 append of a whole fresh block (16 tokens t..t+15 at offsets 0..15 of
 // block blk, block_size 16) for one head, K and V, by one wave -- the prompt
 // case. The block starts afresh (its scale is the run's), so nothing earlier
 // is re-encoded. Returns false, having written nothing, when the block's
-// inputs hold a NaN (the caller then takes fp8_append_run_vec, which codes NaN
+// inputs hold a NaN (the caller then takes fp8_append_run_kv, which codes NaN
 // as e4m3_encode does). K: lane l quantises token l % 16, 16-d chunks
 // l / 16 + 4 j, each one 16-byte store; V: lane l owns d rows RV l .. RV l +
 // RV - 1 (RV = D / 64) and stores each row's 16 tokens as 16 bytes. Each

@@ -136,7 +136,9 @@ __global__ __launch_bounds__(256) void append_bf16_bulk_kernel(uint16_t *__restr
   }
 }
 
-template <int D>
+// One wave per (token, KV head): the first token of a run appends the run.
+// ROWS16: source rows 16-byte aligned, whose runs go as a bulk call's do.
+template <int D, bool ROWS16>
 __global__ __launch_bounds__(64) void append_fp8_kernel(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
                                                         float *__restrict__ ks, float *__restrict__ vs,
                                                         const uint16_t *__restrict__ key, int64_t kst,
@@ -161,6 +163,10 @@ __global__ __launch_bounds__(64) void append_fp8_kernel(uint8_t *__restrict__ kc
     ++r;
   }
   const int first = static_cast<int>(slot % BS);
+  if constexpr (ROWS16) {
+    fp8_append_run_kv<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
+    return;
+  }
   fp8_append_one<D, false>(kc, ks, key, kst, ksh, slots, t, r, blk, first, h, H, BS);
   fp8_append_one<D, true>(vc, vs, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
 }
@@ -179,7 +185,7 @@ __global__ __launch_bounds__(64) void append_fp8_kernel(uint8_t *__restrict__ kc
 // block per wave: 16,384 tokens x 8 heads 23.5 us (one wave per window 23.9,
 // eight 30.1; kernel traces). A whole fresh 16-token block (the prompt case) takes
 // fp8_append_block16: 16-byte loads and stores, hardware code conversion.
-// Other runs: fp8_append_run_vec.
+// Other runs: fp8_append_run_kv.
 constexpr int kFp8BulkMinTokens = 64;
 // Calls of this many tokens or more are taken as prompts (NW = 4), smaller
 // ones as decode-shaped (NW = 8).
@@ -244,8 +250,7 @@ __global__ __launch_bounds__(64 * NW) void append_fp8_bulk_kernel(uint8_t *__res
     if (BS == 16 && first == 0 && r == 16 && __all(slots[t + (lane & 15)] == slot + (lane & 15)) &&
         fp8_append_block16<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, t, blk, h, H))
       continue;
-    fp8_append_run_vec<D, false>(kc, ks, key, kst, ksh, slots, t, r, blk, first, h, H, BS);
-    fp8_append_run_vec<D, true>(vc, vs, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
+    fp8_append_run_kv<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
   }
 }
 
@@ -493,14 +498,18 @@ extern "C" int wkv_append_fp8(const wkv_cache_t *cache, const void *key, int64_t
       if (prompt) WKV_FP8_BULK(64, 4); else WKV_FP8_BULK(64, 8);
     }
 #undef WKV_FP8_BULK
-  } else if (D == 128)
-    append_fp8_kernel<128><<<grid, 64, 0, s>>>(kc, vc, cache->k_scale, cache->v_scale, k, key_stride_t,
-                                               key_stride_h, v, value_stride_t, value_stride_h, slot_mapping,
-                                               num_tokens, H, cache->block_size, cache->num_blocks);
-  else
-    append_fp8_kernel<64><<<grid, 64, 0, s>>>(kc, vc, cache->k_scale, cache->v_scale, k, key_stride_t,
-                                              key_stride_h, v, value_stride_t, value_stride_h, slot_mapping,
-                                              num_tokens, H, cache->block_size, cache->num_blocks);
+  } else {
+#define WKV_FP8_RUNS(Dv, R16)                                                                                      \
+  append_fp8_kernel<Dv, R16><<<grid, 64, 0, s>>>(kc, vc, cache->k_scale, cache->v_scale, k, key_stride_t,          \
+                                                 key_stride_h, v, value_stride_t, value_stride_h, slot_mapping,    \
+                                                 num_tokens, H, cache->block_size, cache->num_blocks)
+    if (D == 128) {
+      if (rows16) WKV_FP8_RUNS(128, true); else WKV_FP8_RUNS(128, false);
+    } else {
+      if (rows16) WKV_FP8_RUNS(64, true); else WKV_FP8_RUNS(64, false);
+    }
+#undef WKV_FP8_RUNS
+  }
   WKV_CHECK_LAUNCH("wkv_append_fp8");
   return WKV_OK;
 }
