@@ -7,9 +7,7 @@
 namespace wkv {
 
 // ---------------------------------------------------------------------------
-// fp8 append of one run (tokens t..t+r-1, all in block blk, the first at
-// offset `first`) for one head, by one wave: scale update, re-encode of the
-// block's earlier entries when the scale grows, then the run's codes.
+// Where element d of the token at offset off lies in the K and V codes.
 template <int D>
 __device__ __forceinline__ int64_t fp8_k_index(int64_t blk, int h, int H, int BS, int off, int d) {
   return (((blk * H + h) * (D / 16) + (d >> 4)) * BS + off) * 16 + (d & 15);
@@ -70,46 +68,6 @@ __device__ __forceinline__ void fp8_reencode_block(uint8_t *__restrict__ cache, 
       base[p] = o;
     }
   }
-}
-
-template <int D, bool IS_V>
-__device__ void fp8_append_one(uint8_t *__restrict__ cache, float *__restrict__ scales,
-                               const uint16_t *__restrict__ src, int64_t st, int64_t sh,
-                               const int64_t *__restrict__ slots, int64_t t, int r, int64_t blk, int first,
-                               int h, int H, int BS) {
-  const int lane = threadIdx.x & 63;  // the calling wave's lane (workgroups may hold several waves)
-  float amax = 0.0f;
-  for (int e = lane; e < r * D; e += 64) {
-    const int tok = e / D, d = e % D;
-    amax = fmaxf(amax, fabsf(bf16_bits_to_f32(src[(t + tok) * st + h * sh + d])));
-  }
-  amax = wave_max(amax);
-  const float s_new = pow2_scale(amax);
-  float s = s_new;
-  if (first != 0) {
-    const float s_old = scales[blk * H + h];
-    s = (s_new > s_old) ? s_new : s_old;
-    if (s > s_old) {
-      // Byte by byte: with fp8_reencode_block here the fused decode kernel that
-      // inlines this (one run of one token) measured 3-4% slower per launch
-      // even in steps where no block grows (fp8 Qwen2.5-7B groups and Qwen3-4B
-      // shapes, in-process A/B).
-      const float ratio = s_old / s;  // exact power of two
-      for (int e = lane; e < first * D; e += 64) {
-        const int off = e / D, d = e % D;
-        const int64_t a = IS_V ? fp8_v_index<D>(blk, h, H, BS, off, d) : fp8_k_index<D>(blk, h, H, BS, off, d);
-        cache[a] = static_cast<uint8_t>(e4m3_encode(e4m3_decode(cache[a]) * ratio));
-      }
-    }
-  }
-  for (int e = lane; e < r * D; e += 64) {
-    const int tok = e / D, d = e % D;
-    const int off = static_cast<int>(slots[t + tok] % BS);
-    const float x = bf16_bits_to_f32(src[(t + tok) * st + h * sh + d]);
-    const int64_t a = IS_V ? fp8_v_index<D>(blk, h, H, BS, off, d) : fp8_k_index<D>(blk, h, H, BS, off, d);
-    cache[a] = static_cast<uint8_t>(e4m3_quantize(x, s));
-  }
-  if (lane == 0) scales[blk * H + h] = s;
 }
 
 // The step token's K and V rows of one head as loaded (bf16 bits, d = lane +
@@ -184,7 +142,10 @@ __device__ __forceinline__ Fp8TokenCodes<D> fp8_token_codes(const float *__restr
 // V together, from its loaded rows: both old scales are loaded at once and
 // both rows reduced side by side, so the two appends cost one chain of memory
 // round trips instead of two. The same codes, scales and re-encodes as
-// fp8_append_one on each of K and V with a run of one token.
+// fp8_append_run_kv with a run of one token. The re-encodes go byte by byte:
+// with fp8_reencode_block in the fused decode kernel that inlines this, a
+// launch measured 3-4% slower even in steps where no block grows (fp8
+// Qwen2.5-7B groups and Qwen3-4B shapes, in-process A/B).
 template <int D>
 __device__ __forceinline__ void fp8_append_token_kv(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
                                                     float *__restrict__ ks, float *__restrict__ vs,
@@ -262,8 +223,9 @@ __device__ __forceinline__ u32x2 e4m3_pack8(uint32_t w0, uint32_t w1, uint32_t w
 }
 
 // fp8 append of one run (tokens t..t+r-1, all in block blk, the first at offset
-// `first`) for one head, K and V together, by one wave: the codes, scales and
-// re-encodes of fp8_append_one. Bound by memory round trips, so the run goes in
+// `first`) for one head, K and V together, by one wave: scale update, re-encode
+// of the block's earlier entries when a scale grows, then the run's codes
+// (e4m3_quantize's). Bound by memory round trips, so the run goes in
 // pieces of 16 tokens whose rows, slots and old scales are all requested before
 // the first is used (K: lane l holds token l % 16, 16-d chunks l / 16 + 4 j; V:
 // RV = D / 64 rows of every token), and a run of one piece -- any run of a

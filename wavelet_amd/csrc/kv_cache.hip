@@ -137,8 +137,7 @@ __global__ __launch_bounds__(256) void append_bf16_bulk_kernel(uint16_t *__restr
 }
 
 // One wave per (token, KV head): the first token of a run appends the run.
-// ROWS16: source rows 16-byte aligned, whose runs go as a bulk call's do.
-template <int D, bool ROWS16>
+template <int D>
 __global__ __launch_bounds__(64) void append_fp8_kernel(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
                                                         float *__restrict__ ks, float *__restrict__ vs,
                                                         const uint16_t *__restrict__ key, int64_t kst,
@@ -163,12 +162,7 @@ __global__ __launch_bounds__(64) void append_fp8_kernel(uint8_t *__restrict__ kc
     ++r;
   }
   const int first = static_cast<int>(slot % BS);
-  if constexpr (ROWS16) {
-    fp8_append_run_kv<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
-    return;
-  }
-  fp8_append_one<D, false>(kc, ks, key, kst, ksh, slots, t, r, blk, first, h, H, BS);
-  fp8_append_one<D, true>(vc, vs, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
+  fp8_append_run_kv<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
 }
 
 // Bulk fp8 append (calls of 64 tokens or more): one workgroup of NW waves per
@@ -481,10 +475,7 @@ extern "C" int wkv_append_fp8(const wkv_cache_t *cache, const void *key, int64_t
   auto vc = static_cast<uint8_t *>(cache->v);
   auto k = static_cast<const uint16_t *>(key);
   auto v = static_cast<const uint16_t *>(value);
-  // 16-byte source rows for the bulk kernel's vector loads
-  const bool rows16 = aligned16(key) && aligned16(value) && key_stride_t % 8 == 0 && key_stride_h % 8 == 0 &&
-                      value_stride_t % 8 == 0 && value_stride_h % 8 == 0;
-  if (num_tokens >= kFp8BulkMinTokens && rows16) {
+  if (num_tokens >= kFp8BulkMinTokens) {
     const dim3 bgrid(static_cast<unsigned>((num_tokens + 63) / 64), static_cast<unsigned>(H));
 #define WKV_FP8_BULK(Dv, NWv)                                                                                   \
   append_fp8_bulk_kernel<Dv, NWv><<<bgrid, 64 * NWv, 0, s>>>(kc, vc, cache->k_scale, cache->v_scale, k,         \
@@ -499,15 +490,11 @@ extern "C" int wkv_append_fp8(const wkv_cache_t *cache, const void *key, int64_t
     }
 #undef WKV_FP8_BULK
   } else {
-#define WKV_FP8_RUNS(Dv, R16)                                                                                      \
-  append_fp8_kernel<Dv, R16><<<grid, 64, 0, s>>>(kc, vc, cache->k_scale, cache->v_scale, k, key_stride_t,          \
-                                                 key_stride_h, v, value_stride_t, value_stride_h, slot_mapping,    \
-                                                 num_tokens, H, cache->block_size, cache->num_blocks)
-    if (D == 128) {
-      if (rows16) WKV_FP8_RUNS(128, true); else WKV_FP8_RUNS(128, false);
-    } else {
-      if (rows16) WKV_FP8_RUNS(64, true); else WKV_FP8_RUNS(64, false);
-    }
+#define WKV_FP8_RUNS(Dv)                                                                                            \
+  append_fp8_kernel<Dv><<<grid, 64, 0, s>>>(kc, vc, cache->k_scale, cache->v_scale, k, key_stride_t, key_stride_h, \
+                                            v, value_stride_t, value_stride_h, slot_mapping, num_tokens, H,        \
+                                            cache->block_size, cache->num_blocks)
+    if (D == 128) WKV_FP8_RUNS(128); else WKV_FP8_RUNS(64);
 #undef WKV_FP8_RUNS
   }
   WKV_CHECK_LAUNCH("wkv_append_fp8");
