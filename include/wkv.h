@@ -133,6 +133,15 @@ int wkv_gather(const wkv_cache_t *cache, const int32_t *block_table, int64_t bt_
                int32_t max_blocks_per_seq, const int32_t *seq_lens, const int64_t *cu_seq_lens,
                int32_t batch, void *out_k, void *out_v, int32_t dequant, void *stream);
 
+/* The same with every sequence's rows after the rows of those before it
+ * (cu_seq_lens[i] = seq_lens[0] + .. + seq_lens[i - 1], added up on the way):
+ * at most WKV_GATHER_PACKED_MAX_BATCH sequences, past which a workgroup's sum
+ * would cost more than a prefix sum made once. */
+#define WKV_GATHER_PACKED_MAX_BATCH 1024
+int wkv_gather_packed(const wkv_cache_t *cache, const int32_t *block_table, int64_t bt_stride,
+                      int32_t max_blocks_per_seq, const int32_t *seq_lens, int32_t batch, void *out_k, void *out_v,
+                      int32_t dequant, void *stream);
+
 /* Copy whole blocks (K, V and fp8 scales): for i < n, block mapping[2i+1]
  * becomes a copy of block mapping[2i]. The pairs are copied concurrently, so
  * they must be independent: no block may be the destination of one pair and

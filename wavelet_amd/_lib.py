@@ -18,6 +18,7 @@ LIB_PATH = Path(__file__).resolve().parent / "libwkv.so"
 WKV_OK, WKV_ERR_INVALID, WKV_ERR_UNSUPPORTED, WKV_ERR_LAUNCH = 0, 1, 2, 3
 WKV_KV_BF16, WKV_KV_FP8_E4M3 = 0, 1
 WKV_NOALLOC_SCRATCH_BYTES = 32 << 20  # include/wkv.h
+WKV_GATHER_PACKED_MAX_BATCH = 1024  # include/wkv.h
 
 
 # wkv_cache_t.flags: several sequences read the same blocks (prefix caching)
@@ -57,6 +58,7 @@ _SIGNATURES = {
     "wkv_mla_append": (c_int, [POINTER(WkvMlaCache), c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
     "wkv_gather": (c_int, [POINTER(WkvCache), c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_void_p]),
     "wkv_copy_blocks": (c_int, [POINTER(WkvCache), c_void_p, c_int64, c_void_p]),
+    "wkv_gather_packed": (c_int, [POINTER(WkvCache), c_void_p, c_int64, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_void_p]),
     "wkv_mla_gather": (c_int, [POINTER(WkvMlaCache), c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_int32, c_void_p, c_void_p]),
     "wkv_mla_copy_blocks": (c_int, [POINTER(WkvMlaCache), c_void_p, c_int64, c_void_p]),
     "wkv_decode_workspace_size": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32]),

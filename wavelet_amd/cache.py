@@ -200,9 +200,6 @@ class PagedKVCache:
         """
         block_table, seq_lens = check_tables(block_table, seq_lens, self.device, self.block_size)
         batch = seq_lens.shape[0]
-        cu = torch.zeros(batch, dtype=torch.int64, device=self.device)
-        if batch > 1:
-            cu[1:] = torch.cumsum(seq_lens[:-1].to(torch.int64), 0)
         total = int(seq_lens.to(torch.int64).sum().item()) if total_tokens is None else int(total_tokens)
         fp8 = self.kv_dtype == "fp8_e4m3"
         if dequant and not fp8:
@@ -213,12 +210,15 @@ class PagedKVCache:
         out_v = torch.empty(shape, dtype=dt, device=self.device)
         if total == 0 or batch == 0:
             return out_k, out_v
-        rc = _lib.load().wkv_gather(
-            ctypes.byref(self.descriptor()),
-            block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
-            seq_lens.data_ptr(), cu.data_ptr(), batch,
-            out_k.data_ptr(), out_v.data_ptr(), int(dequant), _stream(self.device),
-        )
+        table = (ctypes.byref(self.descriptor()), block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
+                 seq_lens.data_ptr())
+        out = (batch, out_k.data_ptr(), out_v.data_ptr(), int(dequant), _stream(self.device))
+        if batch <= _lib.WKV_GATHER_PACKED_MAX_BATCH:
+            rc = _lib.load().wkv_gather_packed(*table, *out)
+        else:
+            cu = torch.zeros(batch, dtype=torch.int64, device=self.device)
+            cu[1:] = torch.cumsum(seq_lens[:-1].to(torch.int64), 0)
+            rc = _lib.load().wkv_gather(*table, cu.data_ptr(), *out)
         _lib.check(rc, "gather")
         return out_k, out_v
 
