@@ -256,10 +256,10 @@ __device__ __forceinline__ int64_t lens_before(const int32_t *__restrict__ lens,
 }
 
 // ---------------------------------------------------------------------------
-// Gather: one workgroup per (sequence, block index). Reads follow the
-// physical order (coalesced); writes are 16-byte pieces of the contiguous
-// [tokens, H, D] output. Bound by HBM: 18,000 tokens of 8 heads (147 MB) take
-// 29 us from the caches, 41 from HBM. cu = nullptr: sequence i starts at the
+// Gather: one workgroup per (sequence, block index), reading whole blocks and
+// writing whole rows of the contiguous [tokens, H, D] output. Bound by HBM: 18,000 tokens of 8 heads (147 MB) take
+// 28 us, inputs in the caches, 34 from HBM (41 with V read an element at a time
+// and K written 16 bytes to a row). cu = nullptr: sequence i starts at the
 // sum of the lengths before it, which each wave adds up itself (a few loads
 // beside the block id's) -- the prefix sum as launches of its own cost the
 // call 7.7 us more.
@@ -283,57 +283,102 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint8_t *__restrict__
   const int ntok = (L - j * BS) < BS ? (L - j * BS) : BS;
   const int64_t tok0 = (cu != nullptr ? cu[i] : lens_before(seq_lens, i)) + static_cast<int64_t>(j) * BS;
 
-  // K: work item = one 16-byte chunk (X elements of one token, one head).
-  for (int w = threadIdx.x; w < H * C * ntok; w += 256) {
-    const int o = w % ntok, hc = w / ntok, c = hc % C, h = hc / C;
-    const u32x4 raw = *reinterpret_cast<const u32x4 *>(kc + ((((blk * H + h) * C + c) * BS + o) * 16));
-    uint8_t *dst = out_k + (((tok0 + o) * H + h) * D + c * X) * OSZ;
-    if constexpr (!DEQUANT) {
-      *reinterpret_cast<u32x4 *>(dst) = raw;
-    } else {
-      const float s = ks[blk * H + h];
-      u32x4 lo, hi;
+  // K: work item = one 16-byte chunk (X elements of one token, one head), the
+  // chunks of a row in consecutive lanes, KB items a thread in flight.
+  constexpr int KB = 4;
+  const int nk = H * C * ntok;
+  for (int w0 = threadIdx.x; w0 < nk; w0 += 256 * KB) {
+    u32x4 raw[KB];
 #pragma unroll
-      for (int q = 0; q < 16; q += 2) {
-        const uint32_t b0 = (raw[q >> 2] >> (8 * (q & 3))) & 0xffu;
-        const uint32_t b1 = (raw[q >> 2] >> (8 * ((q & 3) + 1))) & 0xffu;
-        const uint32_t pk = f32_to_bf16_bits(e4m3_decode(b0) * s) | (f32_to_bf16_bits(e4m3_decode(b1) * s) << 16);
-        if (q < 8) lo[q >> 1] = pk; else hi[(q - 8) >> 1] = pk;
+    for (int k = 0; k < KB; ++k) {
+      const int w = w0 + 256 * k < nk ? w0 + 256 * k : w0;
+      const int c = w % C, ho = w / C, h = ho / ntok, o = ho - h * ntok;
+      raw[k] = *reinterpret_cast<const u32x4 *>(kc + ((((blk * H + h) * C + c) * BS + o) * 16));
+    }
+#pragma unroll
+    for (int k = 0; k < KB; ++k) {
+      const int w = w0 + 256 * k;
+      if (w >= nk) break;
+      const int c = w % C, ho = w / C, h = ho / ntok, o = ho - h * ntok;
+      uint8_t *dst = out_k + (((tok0 + o) * H + h) * D + c * X) * OSZ;
+      if constexpr (!DEQUANT) {
+        *reinterpret_cast<u32x4 *>(dst) = raw[k];
+      } else {
+        const float s = ks[blk * H + h];
+        u32x4 lo, hi;
+#pragma unroll
+        for (int q = 0; q < 16; q += 2) {
+          const uint32_t b0 = (raw[k][q >> 2] >> (8 * (q & 3))) & 0xffu;
+          const uint32_t b1 = (raw[k][q >> 2] >> (8 * ((q & 3) + 1))) & 0xffu;
+          const uint32_t pk = f32_to_bf16_bits(e4m3_decode(b0) * s) | (f32_to_bf16_bits(e4m3_decode(b1) * s) << 16);
+          if (q < 8) lo[q >> 1] = pk; else hi[(q - 8) >> 1] = pk;
+        }
+        reinterpret_cast<u32x4 *>(dst)[0] = lo;
+        reinterpret_cast<u32x4 *>(dst)[1] = hi;
       }
-      reinterpret_cast<u32x4 *>(dst)[0] = lo;
-      reinterpret_cast<u32x4 *>(dst)[1] = hi;
     }
   }
-  // V: work item = 8 consecutive d of one token and head (stride BS in the cache).
-  for (int w = threadIdx.x; w < H * (D / 8) * ntok; w += 256) {
-    const int o = w % ntok, hg = w / ntok, g = hg % (D / 8), h = hg / (D / 8);
-    const int64_t base = ((blk * H + h) * D + g * 8) * BS + o;
-    uint8_t *dst = out_v + (((tok0 + o) * H + h) * D + g * 8) * OSZ;
-    if constexpr (!FP8) {
-      const uint16_t *src = reinterpret_cast<const uint16_t *>(vc);
-      u32x4 pk;
+  // V: tiles of one head's 16 tokens, VT at a time through LDS: read as the
+  // cache holds them (16 tokens of a d row contiguous), in 16-byte pieces, and
+  // written as rows, 16 bytes of a token's d at a time, a row in consecutive
+  // lanes. A d row's pitch in LDS is one dword more than its bytes: the eight
+  // rows of a lane's piece, and those of its neighbours, lie in other banks.
+  constexpr int RB = 16 * ESZ;         // bytes of a d row of a tile
+  constexpr int RP = RB + 4;           // its pitch in LDS
+  constexpr int PR = RB / 16;          // 16-byte pieces of a d row
+  constexpr int VT = 1024 / (D * PR);  // tiles of 1,024 pieces, four per thread
+  constexpr int E = 16 / OSZ;          // elements of an output piece
+  constexpr int PT = 16 * D / E;       // output pieces of a tile
+  __shared__ uint8_t lv[VT * D * RP];
+  const int ng = (ntok + 15) / 16;  // a head's tiles
+  for (int q0 = 0; q0 < H * ng; q0 += VT) {
+    if (q0 > 0) __syncthreads();
+    u32x4 raw[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        pk[q] = static_cast<uint32_t>(src[base + (2 * q) * BS]) | (static_cast<uint32_t>(src[base + (2 * q + 1) * BS]) << 16);
-      *reinterpret_cast<u32x4 *>(dst) = pk;
-    } else if constexpr (!DEQUANT) {
-      u32x2 pk;
+    for (int k = 0; k < 4; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      const int q = q0 + i / (D * PR) < H * ng ? q0 + i / (D * PR) : q0;
+      const int h = q / ng, g = q - h * ng, d = i / PR % D;
+      raw[k] = *reinterpret_cast<const u32x4 *>(vc + (((blk * H + h) * D + d) * BS + 16 * g) * ESZ + 16 * (i % PR));
+    }
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        uint32_t wv = 0;
+    for (int k = 0; k < 4; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      uint32_t *l = reinterpret_cast<uint32_t *>(&lv[(i / PR) * RP + 16 * (i % PR)]);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) wv |= static_cast<uint32_t>(vc[base + (4 * q + b) * BS]) << (8 * b);
-        pk[q] = wv;
+      for (int j = 0; j < 4; ++j) l[j] = raw[k][j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < VT * PT / 256; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      const int t = i / PT, o = i % PT / (D / E), d0 = i % (D / E) * E;
+      const int q = q0 + t;
+      const int h = q / ng, g = q - h * ng;
+      if (q >= H * ng || 16 * g + o >= ntok) continue;
+      uint32_t x[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const uint8_t *l = &lv[(t * D + d0 + e) * RP + o * ESZ];
+        if constexpr (FP8)
+          x[e] = *l;
+        else
+          x[e] = *reinterpret_cast<const uint16_t *>(l);
       }
-      *reinterpret_cast<u32x2 *>(dst) = pk;
-    } else {
-      const float s = vs[blk * H + h];
       u32x4 pk;
+      if constexpr (DEQUANT) {
+        const float s = vs[blk * H + h];
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        pk[q] = f32_to_bf16_bits(e4m3_decode(vc[base + (2 * q) * BS]) * s) |
-                (f32_to_bf16_bits(e4m3_decode(vc[base + (2 * q + 1) * BS]) * s) << 16);
-      *reinterpret_cast<u32x4 *>(dst) = pk;
+        for (int e = 0; e < E; e += 2)
+          pk[e / 2] = f32_to_bf16_bits(e4m3_decode(x[e]) * s) | (f32_to_bf16_bits(e4m3_decode(x[e + 1]) * s) << 16);
+      } else if constexpr (FP8) {
+#pragma unroll
+        for (int e = 0; e < E; e += 4) pk[e / 4] = x[e] | (x[e + 1] << 8) | (x[e + 2] << 16) | (x[e + 3] << 24);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; e += 2) pk[e / 2] = x[e] | (x[e + 1] << 16);
+      }
+      *reinterpret_cast<u32x4 *>(out_v + (((tok0 + 16 * g + o) * H + h) * D + d0) * OSZ) = pk;
     }
   }
 }
