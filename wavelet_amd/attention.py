@@ -66,7 +66,8 @@ def _max_len(seq_lens: torch.Tensor, max_seq_len: int | None) -> int:
 def decode_plan(batch: int, num_kv_heads: int, max_seq_len: int, block_size: int,
                 partition_size: int = 0) -> tuple[int, int, int]:
     """(partition size, waves per workgroup, workgroups per sequence and KV head)
-    that ``paged_decode_gqa`` launches for this geometry (host-side, no GPU)."""
+    that ``paged_decode_gqa`` launches for this geometry (host-side, no GPU). A chosen (.., 4, 2)
+    is launched as one workgroup of eight waves for fp8 or d=64 caches."""
     p, w, c = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
     _lib.check(_lib.load().wkv_decode_plan(int(batch), int(num_kv_heads), int(max_seq_len), int(block_size),
                                            int(partition_size), ctypes.byref(p), ctypes.byref(w), ctypes.byref(c)),

@@ -486,6 +486,30 @@ static void decode_shape(int max_seq, int partition_size, int *W, int *chunks) {
   *chunks = (max_parts + *W - 1) / *W;
 }
 
+// The launch shape when the caller leaves the partition to the library. Narrow
+// rows (256 bytes of K and V per token and head, or less: d=64 bf16, fp8) whose
+// longest context has 5 to 7 partitions take one workgroup of eight waves per
+// sequence and head, an eighth of the longest context each, in the place of two
+// workgroups and a merge launch. 700 tokens, a layer of a captured step, two
+// workgroups -> one: d=64 bf16 2 heads, 1 / 32 / 256 sequences 8.9 / 9.7 / 23.1
+// -> 7.9 / 9.6 / 19.5 us; d=128 fp8 4 heads, the same 10.9 / 12.2 / 45.7 -> 10.2
+// / 11.3 / 39.7 us (520 to 890 tokens alike, mixed lengths more; the first with
+// 32 sequences of 890 tokens alone is slower, 11.0 -> 11.5). Wider rows keep
+// two, as one CU streams no more than about 60 bytes a ns: d=128 bf16 8 heads,
+// 8 sequences 12.0 us in two, 13.7 in one.
+// (Up to 4 partitions, eight waves in the place of four gain 6% for one sequence
+// of 500 tokens and lose 6% for 64.)
+constexpr int kNarrowRowBytes = 256;
+static void choose_shape(int batch, int hkv, int max_seq, int BS, int row_bytes, int *P, int *W, int *chunks) {
+  *P = choose_partition(batch, hkv, max_seq, BS);
+  decode_shape(max_seq, *P, W, chunks);
+  if (row_bytes <= kNarrowRowBytes && *W == 4 && *chunks == 2) {
+    *P = ((max_seq + 7) / 8 + BS - 1) / BS * BS;
+    *W = 8;
+    *chunks = 1;
+  }
+}
+
 }  // namespace wkv
 
 using namespace wkv;
@@ -581,11 +605,8 @@ __global__ __launch_bounds__(256) void decode_order_kernel(const int32_t *__rest
 // 1 (plain longest-first order) when the classes would not be of equal size.
 constexpr int kXcds = 8;
 
-static int grouped_order_classes(int batch, int group_size, int hkv, int max_seq, int BS, int partition_size) {
-  const int P = partition_size != 0 ? partition_size : choose_partition(batch, hkv, max_seq, BS);
-  int W, chunks;
-  decode_shape(max_seq, P, &W, &chunks);
-  int a = chunks * hkv % kXcds, g = kXcds;  // gcd(kXcds, chunks * hkv)
+static int order_classes(int workgroups, int batch, int group_size) {
+  int a = workgroups % kXcds, g = kXcds;  // gcd(kXcds, workgroups)
   while (a != 0) {
     const int t = g % a;
     g = a;
@@ -593,6 +614,20 @@ static int grouped_order_classes(int batch, int group_size, int hkv, int max_seq
   }
   const int n_cls = kXcds / g;
   return batch % (group_size * n_cls) == 0 ? n_cls : 1;
+}
+
+static int grouped_order_classes(int batch, int group_size, int hkv, int max_seq, int BS, int partition_size) {
+  const int P = partition_size != 0 ? partition_size : choose_partition(batch, hkv, max_seq, BS);
+  int W, chunks;
+  decode_shape(max_seq, P, &W, &chunks);
+  if (partition_size == 0 && W == 4 && chunks == 2) {
+    // Two workgroups per sequence and head, or one for narrow rows (choose_shape; the order is
+    // made without the cache): a position's residue modulo the classes of one gives its residue
+    // modulo those of two, so the order of one keeps groups together in both.
+    const int n = order_classes(hkv, batch, group_size);
+    if (n > 1) return n;
+  }
+  return order_classes(chunks * hkv, batch, group_size);
 }
 
 static int launch_decode(const wkv_cache_t *cache, const void *q, int64_t q_stride_b, int64_t q_stride_h, void *out,
@@ -623,15 +658,19 @@ static int launch_decode(const wkv_cache_t *cache, const void *q, int64_t q_stri
   WKV_CHECK_ARG(max_seq_len >= 0, "max_seq_len must be >= 0");
   WKV_CHECK_ARG(std::isfinite(scale), "scale must be finite");
   const int max_seq = max_seq_len < max_blocks_per_seq * BS ? max_seq_len : max_blocks_per_seq * BS;
-  if (partition_size == 0) partition_size = choose_partition(batch, Hkv, max_seq, BS);
+  int W = 0, max_chunks = 0;
+  const bool chosen = partition_size == 0;
+  if (chosen) {
+    const int row_bytes = cache->kv_dtype == WKV_KV_FP8_E4M3 ? 2 * D : 4 * D;
+    choose_shape(batch, Hkv, max_seq, BS, row_bytes, &partition_size, &W, &max_chunks);
+  }
   WKV_CHECK_ARG(partition_size >= 16 && partition_size % 16 == 0, "partition_size must be a positive multiple of 16");
   WKV_CHECK_ARG((partition_size + BS - 17) / BS + 1 <= 64,
                 "partition_size %d spans more than 64 blocks of %d tokens", partition_size, BS);
   if (ap != nullptr)
     WKV_CHECK_ARG(partition_size % BS == 0, "a fused append needs partition_size %d to be a multiple of block_size %d",
                   partition_size, BS);
-  int W, max_chunks;
-  decode_shape(max_seq, partition_size, &W, &max_chunks);
+  if (!chosen) decode_shape(max_seq, partition_size, &W, &max_chunks);
   WKV_CHECK_ARG(max_chunks <= 65535, "too many partitions");
   const int64_t need = wkv_decode_workspace_size(batch, num_q_heads, D, max_seq, partition_size * W);
   if (max_chunks > 1 && static_scratch)
