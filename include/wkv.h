@@ -223,8 +223,11 @@ int wkv_grouped_decode_order(const int32_t *seq_lens, int32_t batch, int32_t gro
  * only, no GPU): the partition size (partition_size, or the library's choice
  * when 0), the waves per workgroup and the workgroups (chunks) per sequence
  * and KV head; more than one chunk leaves partials for the merge kernel. (The
- * library's choice of two chunks of four waves is launched as one of eight
- * for fp8 or d=64 caches.) For planning and labelling; no reference counterpart. max_seq_len is the one
+ * library's choice is adapted to the cache and the chip at the launch: two
+ * chunks of four waves go as one of eight for fp8 or d=64 caches, several
+ * chunks of eight waves that would leave CUs idle as more chunks of four;
+ * one chunk never becomes several, and the workspace need stays within
+ * wkv_decode_workspace_size of partition 0.) For planning and labelling; no reference counterpart. max_seq_len is the one
  * the decode call will get, clipped to the block-table width. */
 int wkv_decode_plan(int32_t batch, int32_t num_kv_heads, int32_t max_seq_len, int32_t block_size,
                     int32_t partition_size, int32_t *out_partition, int32_t *out_waves, int32_t *out_chunks);

@@ -1,4 +1,4 @@
-"""Decode over 5 to 7 chosen partitions of narrow rows: one workgroup of eight waves, against the oracle."""
+"""Decode at the edges of the launch shapes the library chooses by size, against the oracle."""
 
 from __future__ import annotations
 
@@ -17,11 +17,33 @@ BF16 = torch.bfloat16
 @pytest.mark.parametrize("top", [512, 513, 700, 896, 897, 1023])
 @pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (32, 8, 128)])
 def test_contexts_around_the_single_workgroup_range(cuda, hq, hkv, d, top, bs):
-    """The longest context at both ends of the range and past them, with contexts of one token, of
+    """Narrow rows of 5 to 7 partitions: the longest context at both ends of the range and past them, with contexts of one token, of
     less than a wave's share and none at all beside it; the same step with the partition given
     (two workgroups and a merge) agrees. d=128 bf16 keeps the two."""
     lens = np.array([top, 1, 0, 15, top // 8, top // 8 + 1, 511, top - 1])
-    w = synth.make_decode_workload(f"narrow{d}t{top}b{bs}", batch=len(lens), num_kv_heads=hkv, num_q_heads=hq,
+    _check(cuda, hq, hkv, d, bs, lens)
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs,lens", [
+    (32, 8, 128, 16, [1024]),  # one workgroup per sequence and head
+    (32, 8, 128, 16, [1025]),  # spread: partitions of 64, four waves
+    (32, 8, 128, 64, [2048, 1, 257, 0]),
+    (32, 8, 128, 16, [2049, 513, 16]),  # spread: partitions of 128
+    (14, 2, 64, 32, [1999, 2048, 255, 1024, 1025]),
+    (14, 2, 64, 16, [4096, 33]),  # eight slots, narrow
+    (14, 2, 64, 16, [4097, 2048]),  # nine: not spread
+    (32, 8, 128, 128, [1500, 300]),
+    (28, 4, 128, 16, [8192] * 4 + [700]),  # 5 x 4 heads x 16 slots: more than one per CU
+])
+def test_few_long_contexts_spread_over_the_chip(cuda, hq, hkv, d, bs, lens):
+    """Both sides of each bound of the rule that spreads few long contexts over more, smaller
+    workgroups; the given partition agrees."""
+    _check(cuda, hq, hkv, d, bs, np.array(lens))
+
+
+def _check(cuda, hq, hkv, d, bs, lens):
+    top = int(lens.max())
+    w = synth.make_decode_workload(f"shape{d}t{top}b{bs}", batch=len(lens), num_kv_heads=hkv, num_q_heads=hq,
                                    head_dim=d, block_size=bs, context_lens=lens)
     gen = np.random.default_rng(top)
     kc, vc = paged.empty_cache(w.num_blocks, bs, hkv, d)

@@ -66,8 +66,9 @@ def _max_len(seq_lens: torch.Tensor, max_seq_len: int | None) -> int:
 def decode_plan(batch: int, num_kv_heads: int, max_seq_len: int, block_size: int,
                 partition_size: int = 0) -> tuple[int, int, int]:
     """(partition size, waves per workgroup, workgroups per sequence and KV head)
-    that ``paged_decode_gqa`` launches for this geometry (host-side, no GPU). A chosen (.., 4, 2)
-    is launched as one workgroup of eight waves for fp8 or d=64 caches."""
+    that ``paged_decode_gqa`` launches for this geometry (host-side, no GPU). The launch adapts
+    a chosen shape to the cache and the chip (include/wkv.h): (.., 4, 2) to one workgroup of eight waves for
+    narrow rows, several workgroups of eight waves to more of four for few sequences."""
     p, w, c = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
     _lib.check(_lib.load().wkv_decode_plan(int(batch), int(num_kv_heads), int(max_seq_len), int(block_size),
                                            int(partition_size), ctypes.byref(p), ctypes.byref(w), ctypes.byref(c)),

@@ -486,6 +486,34 @@ static void decode_shape(int max_seq, int partition_size, int *W, int *chunks) {
   *chunks = (max_parts + *W - 1) / *W;
 }
 
+// Few long contexts, where the chosen shape (partitions of the smallest size,
+// eight waves, several workgroups per sequence and head) would leave CUs without
+// a workgroup: workgroups of four waves while they number at most one per CU,
+// and partitions of 64 tokens up to 2,048. A CU alone streams about 60 bytes a
+// ns however many waves it has, so such a launch lasts as long as its longest
+// workgroup's tokens; half as many per workgroup cost only merge slots. Per
+// layer of a captured step, eight waves -> four: d=128 bf16 8 heads, 1 sequence
+// of 1,500 / 4,000 / 8,000 tokens 15.2 / 19.1 / 20.9 -> 11.7 / 14.6 / 17.6 us, 3
+// of 4,000 20.3 -> 16.5, 8 of 2,048 22.2 -> 18.6; past one per CU it turns (3 of
+// 8,000 24.4 -> 27.9). d=128 fp8 4 heads, 1 of 2,048 / 4,000 15.8 / 14.7 -> 13.5 /
+// 13.9; narrow rows stop gaining at more than 8 slots (1 of 16,000 20.0 -> 20.9).
+// Launches of one workgroup per sequence and head need no scratch and stay.
+constexpr int kDecodeCus = 256;
+constexpr int kNarrowRowBytes = 256;  // K and V of a token and head: d=64 bf16, fp8
+static void spread_shape(int64_t items, int max_seq, int BS, bool narrow, int *P, int *W, int *chunks) {
+  if (*W != 8 || *chunks < 2 || *P != (128 + BS - 1) / BS * BS) return;
+  const int half = (64 + BS - 1) / BS * BS;
+  const int ch = (max_seq + 4 * half - 1) / (4 * half), c = (max_seq + 4 * *P - 1) / (4 * *P);
+  if (max_seq <= 2048 && items * ch <= kDecodeCus) {
+    *P = half;
+    *W = 4;
+    *chunks = ch;
+  } else if (items * c <= kDecodeCus && (!narrow || c <= 8)) {
+    *W = 4;
+    *chunks = c;
+  }
+}
+
 // The launch shape when the caller leaves the partition to the library. Narrow
 // rows (256 bytes of K and V per token and head, or less: d=64 bf16, fp8) whose
 // longest context has 5 to 7 partitions take one workgroup of eight waves per
@@ -499,15 +527,17 @@ static void decode_shape(int max_seq, int partition_size, int *W, int *chunks) {
 // 8 sequences 12.0 us in two, 13.7 in one.
 // (Up to 4 partitions, eight waves in the place of four gain 6% for one sequence
 // of 500 tokens and lose 6% for 64.)
-constexpr int kNarrowRowBytes = 256;
 static void choose_shape(int batch, int hkv, int max_seq, int BS, int row_bytes, int *P, int *W, int *chunks) {
   *P = choose_partition(batch, hkv, max_seq, BS);
   decode_shape(max_seq, *P, W, chunks);
-  if (row_bytes <= kNarrowRowBytes && *W == 4 && *chunks == 2) {
+  const bool narrow = row_bytes <= kNarrowRowBytes;
+  if (narrow && *W == 4 && *chunks == 2) {
     *P = ((max_seq + 7) / 8 + BS - 1) / BS * BS;
     *W = 8;
     *chunks = 1;
+    return;
   }
+  spread_shape(static_cast<int64_t>(batch) * hkv, max_seq, BS, narrow, P, W, chunks);
 }
 
 }  // namespace wkv
@@ -617,10 +647,12 @@ static int order_classes(int workgroups, int batch, int group_size) {
 }
 
 static int grouped_order_classes(int batch, int group_size, int hkv, int max_seq, int BS, int partition_size) {
-  const int P = partition_size != 0 ? partition_size : choose_partition(batch, hkv, max_seq, BS);
+  int P = partition_size != 0 ? partition_size : choose_partition(batch, hkv, max_seq, BS);
   int W, chunks;
   decode_shape(max_seq, P, &W, &chunks);
-  if (partition_size == 0 && W == 4 && chunks == 2) {
+  if (partition_size == 0 && W == 8) {
+    spread_shape(static_cast<int64_t>(batch) * hkv, max_seq, BS, true, &P, &W, &chunks);
+  } else if (partition_size == 0 && W == 4 && chunks == 2) {
     // Two workgroups per sequence and head, or one for narrow rows (choose_shape; the order is
     // made without the cache): a position's residue modulo the classes of one gives its residue
     // modulo those of two, so the order of one keeps groups together in both.
