@@ -329,7 +329,7 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint8_t *__restrict__
   constexpr int VT = 1024 / (D * PR);  // tiles of 1,024 pieces, four per thread
   constexpr int E = 16 / OSZ;          // elements of an output piece
   constexpr int PT = 16 * D / E;       // output pieces of a tile
-  __shared__ uint8_t lv[VT * D * RP];
+  __shared__ __attribute__((aligned(16))) uint8_t lv[VT * D * RP];
   const int ng = (ntok + 15) / 16;  // a head's tiles
   for (int q0 = 0; q0 < H * ng; q0 += VT) {
     if (q0 > 0) __syncthreads();
