@@ -65,7 +65,8 @@ def sample_row(logits, *, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repeti
     """One row -> (token, processed logprob, kept bool mask, ambiguous).
 
     ``ambiguous`` flags a top-p boundary within 1e-6 of the target mass, where
-    a one-ulp difference in exp could move the threshold.
+    a one-ulp difference in exp could move the threshold. A +inf maximum weighs 1 (as a
+    finite one does) and the other tokens of its row nothing; its logprob is inf - inf = NaN.
     """
     l = np.asarray(logits, dtype=np.float32).copy()
     pen = np.float32(repetition_penalty)
@@ -76,10 +77,12 @@ def sample_row(logits, *, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repeti
     greedy = t < GREEDY_EPS
     inv_t = np.float32(1.0) if greedy else np.float32(1.0) / t
     x = (l * inv_t).astype(np.float32)
-    finite = np.isfinite(x)
-    if not finite.any():
+    real = x > -np.inf  # NaN is not
+    if not real.any():
         return 0, -np.inf, np.zeros(x.shape, bool), False
-    mx = np.float32(x[finite].max())
+    mx = np.float32(x[real].max())
+    with np.errstate(invalid="ignore"):
+        below = np.where(x == mx, np.float32(0.0), x - mx).astype(np.float32)
     keys = order_key(x)
     key_lo = order_key(np.float32(-3.402823466e38))
     if min_p > 0:  # (capped at the maximum's key: min_p above 1 still keeps the maximum)
@@ -93,7 +96,7 @@ def sample_row(logits, *, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repeti
     tp = np.float32(top_p)
     if tp < np.float32(1.0):
         kept = keys >= key_lo
-        w = (np.exp((x[kept] - mx).astype(np.float32)).astype(np.float32) * np.float32(4294967296.0)).astype(np.uint64)
+        w = (np.exp(below[kept]).astype(np.float32) * np.float32(4294967296.0)).astype(np.uint64)
         total = int(w.sum(dtype=np.uint64))
         target = int(np.ceil(np.float64(tp) * np.float64(total)))
         kk = keys[kept]
@@ -115,12 +118,13 @@ def sample_row(logits, *, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repeti
             cum += mass[key]
         key_lo = max(key_lo, tau)
     kept = keys >= key_lo
-    z = np.exp((x[kept] - mx).astype(np.float32)).astype(np.float64).sum()
+    z = np.exp(below[kept]).astype(np.float64).sum()
     idx = np.nonzero(kept)[0]
     if greedy:
         score = x[idx]
     else:
         score = (x[idx] - log_exp_variates(seed, step, v)[idx]).astype(np.float32)
     tok = int(idx[np.argmax(score)])  # argmax returns the first (lowest index) maximum
-    logprob = float(np.float64(x[tok] - mx) - np.log(z))
+    with np.errstate(invalid="ignore"):
+        logprob = float(np.float64(x[tok] - mx) - np.log(z))
     return tok, logprob, kept, ambiguous

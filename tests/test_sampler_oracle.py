@@ -107,6 +107,18 @@ def test_min_p_above_one_keeps_the_maximum():
     assert tok in (1, 3) and abs(lp - np.log(0.5)) < 1e-6
 
 
+@pytest.mark.parametrize("kw", [dict(), dict(temperature=0.0), dict(top_k=2), dict(top_p=0.9), dict(min_p=0.1),
+                                dict(top_k=3, top_p=0.5, min_p=0.1)])
+def test_infinite_maximum_wins_every_draw(kw):
+    """+inf beats any finite score and ties go to the lowest index; under top_p and min_p the infinite
+    logits alone are kept (any finite one weighs e^-inf = 0 against them); logprob inf - inf."""
+    x = np.array([0.5, -np.inf, np.inf, 3e38, np.nan, np.inf, -2.0], np.float32)
+    tok, lp, kept, amb = S.sample_row(x, seed=1, step=2, **kw)
+    everything = not ({"top_k", "top_p", "min_p"} & set(kw))
+    assert tok == 2 and np.isnan(lp) and not amb
+    np.testing.assert_array_equal(kept, np.isfinite(x) | (x == np.inf) if everything else x == np.inf)
+
+
 @pytest.mark.parametrize("kw", [dict(min_p=1.5), dict(min_p=-0.1), dict(top_p=0.0), dict(top_p=1.2),
                                 dict(temperature=-1.0), dict(repetition_penalty=0.0)])
 def test_sample_rejects_out_of_range_scalars(kw):

@@ -299,10 +299,12 @@ constexpr int kQueue = 128;
 constexpr int kFastQueue = 64 + 4 * 64;
 static_assert(kBins == 2 * kSampleThreads, "the threshold scan gives every thread two bins");
 
-// e^(x - mx) in units of 2^-32, truncated; x <= mx, so at most 2^32.
+// e^(x - mx) in units of 2^-32, truncated; x <= mx, so at most 2^32. (An
+// infinite maximum, where x - mx is NaN, weighs what a finite one does; every
+// other token of its row then weighs 0.)
 __device__ __forceinline__ unsigned long long fixed_mass(float x, float mx) {
   const float v = expf(x - mx) * 4294967296.f;
-  return v >= 4294967296.f ? 1ull << 32 : static_cast<unsigned long long>(static_cast<uint32_t>(v));
+  return v < 4294967296.f ? static_cast<unsigned long long>(static_cast<uint32_t>(v)) : 1ull << 32;
 }
 
 struct SampleArgs {
@@ -727,8 +729,9 @@ __global__ __launch_bounds__(64) void sample_join_kernel(const T *__restrict__ l
   const int cnt = wave_reduce(on ? sr.cnt[lane] : 0, [](int x, int y) { return x + y; });
   if (lane == 0) {
     const Row<T> row(logits, row_stride, vocab, a, b);
-    a.tokens[b] = bi;
-    if (a.logprobs) a.logprobs[b] = (row.x_of(bi) - mx) - logf(z);
+    const bool drawn = bi < vocab;
+    a.tokens[b] = drawn ? bi : 0;
+    if (a.logprobs) a.logprobs[b] = drawn ? (row.x_of(bi) - mx) - logf(z) : -INFINITY;
     if (a.counts) a.counts[b] = cnt;
   }
 }
@@ -899,7 +902,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
     // bin_of forms it (d >= 0: x <= mx; NaN and -inf fail every compare),
     // bin <= bcap <=> d < bcap + 1 and bin < kMassBins <=> d < kMassBins
     // (bcap + 1 <= kBins - 1). The bin is formed only for the few tokens taken.
-    const bool captured = want_m || bcap < kBins - 1;
+    // A row with an infinite maximum has no distances (inf - inf is NaN, which no
+    // range holds): the key alone decides there, over the whole row.
+    const bool captured = mx < INFINITY && (want_m || bcap < kBins - 1);
     const float bcap1 = want_m ? INFINITY : static_cast<float>(bcap + 1);
     if (captured && use_g) {
       // The groups whose maximum is in the range, four lanes (one chunk each) per group.
@@ -937,7 +942,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
         }
         __syncthreads();
         n = ncand;
-        listed = n <= kCand;
+        listed = n > 0 && n <= kCand;
       }
       __syncthreads();
     } else if (captured) {
@@ -991,7 +996,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
       }
       __syncthreads();
       n = ncand;
-      listed = n <= kCand;
+      listed = n > 0 && n <= kCand;
       mtot = sel_n;
       if (!listed) {  // the list's own tokens join the histogram
         for (int i = tid; i < kCand; i += kSampleThreads) {
@@ -1334,8 +1339,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
   block_argmax(race.best, race.bi, redv, redi);
   const float c = block_sum(static_cast<float>(cnt), redv);
   if (tid == 0) {
-    a.tokens[b] = race.bi;
-    if (a.logprobs) a.logprobs[b] = (row.x_of(race.bi) - mx) - lz;
+    const bool drawn = race.bi < vocab;  // (the maximum is always kept; no index past the row is ever read)
+    a.tokens[b] = drawn ? race.bi : 0;
+    if (a.logprobs) a.logprobs[b] = drawn ? (row.x_of(race.bi) - mx) - lz : -INFINITY;
     if (a.counts) a.counts[b] = static_cast<int32_t>(c);
   }
 }
