@@ -20,6 +20,16 @@ def test_runs_match_oracle(cuda, d, bs, short):
     at offset 0 and inside a block, over earlier codes that hold every e4m3 pattern (NaN codes and
     both zeros among them) under scales that grow and scales that do not, tokens in reverse slot
     order, NaN and infinities in some rows; calls below and above 64 tokens (both launch shapes)."""
+    _check(cuda, d, bs, short, 64)
+
+
+@pytest.mark.parametrize("d,bs", [(64, 16), (128, 16), (128, 64)])
+def test_runs_of_a_prompt_sized_call_match_oracle(cuda, d, bs):
+    """The same runs in one call of 4,096 tokens (skipped slots make up the number): the prompt launch."""
+    _check(cuda, d, bs, False, 4096)
+
+
+def _check(cuda, d, bs, short, pad):
     nb, h = 64, 2
     rng = np.random.default_rng(d + bs + short)
     kc, vc = paged.empty_cache(nb, bs, h, d, dtype=np.uint8, fill=0)
@@ -39,7 +49,7 @@ def test_runs_match_oracle(cuda, d, bs, short):
                 calls.append(next(blocks) * bs + first + np.arange(n))
     calls.append(next(blocks) * bs + np.arange(bs)[::-1])
     if not short:
-        calls = [np.concatenate(calls + [np.full(64, -1)])]
+        calls = [np.concatenate(calls + [np.full(pad, -1)])]
     for i, slots in enumerate(calls):
         slots = slots.astype(np.int64)
         assert (len(slots) >= 64) == (not short) or len(slots) == 64

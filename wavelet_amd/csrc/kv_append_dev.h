@@ -38,10 +38,13 @@ __device__ __forceinline__ uint32_t fp8x4_rescale(uint32_t c, float ratio) {
 // round trip per byte). K [D/16][BS][16]: piece p holds token p % BS's 16
 // d-values of one chunk; V [D][BS]: piece p holds tokens 16 (p % (BS/16)) ..
 // + 15 of one d row. Pieces at or past `first` are not stored.
-template <int D, bool IS_V>
+// LEAN: nothing that depends on the lane is held across a caller's loop over
+// runs (the registers it saves there are worth more than forming it again).
+template <int D, bool IS_V, bool LEAN = false>
 __device__ __forceinline__ void fp8_reencode_block(uint8_t *__restrict__ cache, int64_t blk, int h, int H, int BS,
                                                    int first, float ratio) {
-  const int lane = threadIdx.x & 63;
+  int lane = threadIdx.x & 63;
+  if constexpr (LEAN) asm volatile("" : "+v"(lane));
   u32x4 *base = reinterpret_cast<u32x4 *>(cache + (blk * H + h) * static_cast<int64_t>(D) * BS);
   const int np = D * BS / 16;
   constexpr int PL = 4;
@@ -138,15 +141,15 @@ __device__ __forceinline__ Fp8TokenCodes<D> fp8_token_codes(const float *__restr
   return c;
 }
 
-// fp8 append of one token (the fused decode's step token) for one head, K and
-// V together, from its loaded rows: both old scales are loaded at once and
-// both rows reduced side by side, so the two appends cost one chain of memory
-// round trips instead of two. The same codes, scales and re-encodes as
-// fp8_append_run_kv with a run of one token. The re-encodes go byte by byte:
-// with fp8_reencode_block in the fused decode kernel that inlines this, a
-// launch measured 3-4% slower even in steps where no block grows (fp8
-// Qwen2.5-7B groups and Qwen3-4B shapes, in-process A/B).
-template <int D>
+// fp8 append of one token (the fused decode's step token, a run of one token)
+// for one head, K and V together, from its loaded rows: both old scales are
+// loaded at once and both rows reduced side by side, so the two appends cost
+// one chain of memory round trips instead of two. The same codes, scales and
+// re-encodes as fp8_append_run_kv with a run of one token. PIECES: re-encodes
+// by fp8_reencode_block, else byte by byte: with the former in the fused decode
+// kernel that inlines this, a launch measured 3-4% slower even in steps where
+// no block grows (fp8 Qwen2.5-7B groups and Qwen3-4B shapes, in-process A/B).
+template <int D, bool PIECES = false>
 __device__ __forceinline__ void fp8_append_token_kv(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
                                                     float *__restrict__ ks, float *__restrict__ vs,
                                                     const Fp8TokenRows<D> &rows, int64_t blk, int off, int h, int H,
@@ -171,8 +174,11 @@ __device__ __forceinline__ void fp8_append_token_kv(uint8_t *__restrict__ kc, ui
   av = wave_max(av);
   float sk = pow2_scale(ak), sv = pow2_scale(av);
   if (off != 0) {
-    if (sk > sk_old) {  // the block's earlier K codes at the grown scale, byte by byte
+    if (sk > sk_old) {  // the block's earlier K codes at the grown scale
       const float ratio = sk_old / sk;
+      if constexpr (PIECES)
+        fp8_reencode_block<D, false>(kc, blk, h, H, BS, off, ratio);
+      else
       for (int e = lane; e < off * D; e += 64) {
         const int64_t a = fp8_k_index<D>(blk, h, H, BS, e / D, e % D);
         kc[a] = static_cast<uint8_t>(e4m3_encode(e4m3_decode(kc[a]) * ratio));
@@ -182,6 +188,9 @@ __device__ __forceinline__ void fp8_append_token_kv(uint8_t *__restrict__ kc, ui
     }
     if (sv > sv_old) {
       const float ratio = sv_old / sv;
+      if constexpr (PIECES)
+        fp8_reencode_block<D, true>(vc, blk, h, H, BS, off, ratio);
+      else
       for (int e = lane; e < off * D; e += 64) {
         const int64_t a = fp8_v_index<D>(blk, h, H, BS, e / D, e % D);
         vc[a] = static_cast<uint8_t>(e4m3_encode(e4m3_decode(vc[a]) * ratio));
@@ -235,14 +244,17 @@ __device__ __forceinline__ u32x2 e4m3_pack8(uint32_t w0, uint32_t w1, uint32_t w
 // ragged runs over partly filled blocks, 4 heads: 22.7 us with K and V one
 // after the other and V a token at a time, 11.1 us so. Source rows 16-byte
 // aligned (the host checks).
-template <int D>
-__device__ void fp8_append_run_kv(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc, float *__restrict__ ks,
-                                  float *__restrict__ vs, const uint16_t *__restrict__ key, int64_t kst, int64_t ksh,
-                                  const uint16_t *__restrict__ val, int64_t vst, int64_t vsh,
-                                  const int64_t *__restrict__ slots, int64_t t, int r, int64_t blk, int first, int h,
-                                  int H, int BS) {
+template <int D, bool LEAN>
+__device__ __forceinline__ void fp8_append_run_body(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
+                                                    float *__restrict__ ks, float *__restrict__ vs,
+                                                    const uint16_t *__restrict__ key, int64_t kst, int64_t ksh,
+                                                    const uint16_t *__restrict__ val, int64_t vst, int64_t vsh,
+                                                    const int64_t *__restrict__ slots, int64_t t, int r, int64_t blk,
+                                                    int first, int h, int H, int BS) {
   constexpr int P = 16, NC = D / 64, RV = D / 64;
-  const int lane = threadIdx.x & 63, m = lane & 15;
+  int lane = threadIdx.x & 63;
+  if constexpr (LEAN) asm volatile("" : "+v"(lane));
+  const int m = lane & 15;
   const int64_t si = blk * H + h;
   const float sk_old = first != 0 ? ks[si] : 0.f, sv_old = first != 0 ? vs[si] : 0.f;
   u32x4 kw[NC][2];
@@ -292,11 +304,11 @@ __device__ void fp8_append_run_kv(uint8_t *__restrict__ kc, uint8_t *__restrict_
   float sk = pow2_scale(__uint_as_float(ka << 16)), sv = pow2_scale(__uint_as_float(va << 16));
   if (first != 0) {  // the block's earlier codes are re-encoded at a grown scale (exact power-of-two ratio)
     if (sk > sk_old)
-      fp8_reencode_block<D, false>(kc, blk, h, H, BS, first, sk_old / sk);
+      fp8_reencode_block<D, false, LEAN>(kc, blk, h, H, BS, first, sk_old / sk);
     else
       sk = sk_old;
     if (sv > sv_old)
-      fp8_reencode_block<D, true>(vc, blk, h, H, BS, first, sv_old / sv);
+      fp8_reencode_block<D, true, LEAN>(vc, blk, h, H, BS, first, sv_old / sv);
     else
       sv = sv_old;
   }
@@ -345,6 +357,18 @@ __device__ void fp8_append_run_kv(uint8_t *__restrict__ kc, uint8_t *__restrict_
     ks[si] = sk;
     vs[si] = sv;
   }
+}
+
+// The same for callers without a register target: compiled on its own before it
+// is inlined, it comes out 5 to 10% faster (d=64, runs of 63 tokens in blocks of 64: 19.8 us
+// against 21.3) with 199 registers in the place of some 90.
+template <int D>
+__device__ void fp8_append_run_kv(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc, float *__restrict__ ks,
+                                  float *__restrict__ vs, const uint16_t *__restrict__ key, int64_t kst, int64_t ksh,
+                                  const uint16_t *__restrict__ val, int64_t vst, int64_t vsh,
+                                  const int64_t *__restrict__ slots, int64_t t, int r, int64_t blk, int first, int h,
+                                  int H, int BS) {
+  fp8_append_run_body<D, false>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
 }
 
 // fp8 append of a whole fresh block (16 tokens t..t+15 at offsets 0..15 of

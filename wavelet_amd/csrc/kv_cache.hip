@@ -162,6 +162,12 @@ __global__ __launch_bounds__(64) void append_fp8_kernel(uint8_t *__restrict__ kc
     ++r;
   }
   const int first = static_cast<int>(slot % BS);
+  if (r == 1) {  // (a decode step's token: 3.7 us for one of 8 heads of 128, 5.4 as a run's piece of 16)
+    Fp8TokenRows<D> rows;
+    fp8_token_rows_load<D>(rows, key + t * kst + h * ksh, val + t * vst + h * vsh);
+    fp8_append_token_kv<D, true>(kc, vc, ks, vs, rows, blk, first, h, H, BS);
+    return;
+  }
   fp8_append_run_kv<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
 }
 
@@ -179,13 +185,15 @@ __global__ __launch_bounds__(64) void append_fp8_kernel(uint8_t *__restrict__ kc
 // block per wave: 16,384 tokens x 8 heads 23.5 us (one wave per window 23.9,
 // eight 30.1; kernel traces). A whole fresh 16-token block (the prompt case) takes
 // fp8_append_block16: 16-byte loads and stores, hardware code conversion.
-// Other runs: fp8_append_run_kv.
+// Other runs: fp8_append_run_kv. At d=128 four waves per SIMD (128 registers) are
+// asked for: at two, as the compiler has it otherwise (212), 16,384 tokens x 8
+// heads in whole blocks take 24.2 us in the place of 20.2 (d=64: 5.6 at either).
 constexpr int kFp8BulkMinTokens = 64;
 // Calls of this many tokens or more are taken as prompts (NW = 4), smaller
 // ones as decode-shaped (NW = 8).
 constexpr int64_t kFp8PromptTokens = 4096;
 template <int D, int NW>
-__global__ __launch_bounds__(64 * NW) void append_fp8_bulk_kernel(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
+__global__ __launch_bounds__(64 * NW, D == 128 ? 4 : 1) void append_fp8_bulk_kernel(uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
                                                              float *__restrict__ ks, float *__restrict__ vs,
                                                              const uint16_t *__restrict__ key, int64_t kst,
                                                              int64_t ksh, const uint16_t *__restrict__ val,
@@ -244,7 +252,10 @@ __global__ __launch_bounds__(64 * NW) void append_fp8_bulk_kernel(uint8_t *__res
     if (BS == 16 && first == 0 && r == 16 && __all(slots[t + (lane & 15)] == slot + (lane & 15)) &&
         fp8_append_block16<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, t, blk, h, H))
       continue;
-    fp8_append_run_kv<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
+    if constexpr (D == 128)
+      fp8_append_run_body<D, true>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
+    else
+      fp8_append_run_kv<D>(kc, vc, ks, vs, key, kst, ksh, val, vst, vsh, slots, t, r, blk, first, h, H, BS);
   }
 }
 
