@@ -36,6 +36,19 @@ def test_whole_rows_match_oracle(cuda, whole_rows, vocab, dtype):
     _check_rows(cuda, x, ROWS, seen_lists, np.arange(B, dtype=np.int64) * 1000 + 17, 5, dtype)
 
 
+@pytest.mark.parametrize("vocab", [8192, 8193, 32001])
+def test_list_lengths_around_the_ranked_select(cuda, vocab):
+    """Lists of 127 to 257 entries under top_k alone (ranked up to 128, then by radix) and under top_k and
+    top_p together (up to 256), with ties at the threshold; min_p alone below and above one chunk per thread."""
+    rows = [(1.0, k, p, 0.0, 1.0) for k in (100, 127, 128, 129, 255, 256, 257) for p in (1.0, 0.9)]
+    rows += [(1.0, 0, 1.0, 0.3, 1.0), (0.7, 0, 1.0, 1e-4, 1.2), (1.0, 0, 0.99, 0.0, 1.0), (1.0, 0, 0.9999, 0.0, 1.0)]
+    x = (synth.normal(synth.stream_key("smpr", vocab), len(rows) * vocab) * 4.0).astype(np.float32).reshape(len(rows), vocab)
+    x[::3] = np.round(x[::3] * 16) / 16  # ties
+    rng = np.random.default_rng(vocab)
+    _check_rows(cuda, x, rows, [rng.integers(0, vocab, 64) for _ in rows], np.arange(len(rows), dtype=np.int64) * 7 + 1,
+                3, torch.float32)
+
+
 # (temperature, top_k, top_p, min_p, repetition_penalty): every path of a row, and k at and past the
 # number of waves of the slices
 MIX = ROWS + [(1.0, 300, 1.0, 0.0, 1.0), (1.0, 5000, 0.9, 0.0, 1.0), (0.0, 50, 1.0, 0.0, 1.0), (1.0, 0, 0.999, 0.0, 1.0),
