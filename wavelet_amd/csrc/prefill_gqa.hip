@@ -140,22 +140,23 @@ struct PrefillGrid {
   int W;        // workgroups that share the steps evenly; 0: a workgroup per unit group
   int batch;
   int log2R;
-  FastDiv by_G, by_ug, by_inner, by_Hkv;  // query heads per KV head, n_ug, n_inner, KV heads
+  int G;                                  // query heads per KV head
+  FastDiv by_U, by_ug, by_inner, by_Hkv;  // units per query tile (G, or more: prefill_grid), n_ug, n_inner, KV heads
 };
 
 // The units and 64-key steps of unit group ug of a sequence (uniform).
 struct PrefillRange {
-  int units;    // query heads x query tiles of 32 of the sequence
+  int units;    // units per tile x query tiles of 32 of the sequence
   int kend;     // keys [0, kend) of the group's last query
   int n_steps;  // 64-key steps over them
 };
 
-__device__ __forceinline__ PrefillRange prefill_range(int qlen, int L, const FastDiv &G, int ug) {
+__device__ __forceinline__ PrefillRange prefill_range(int qlen, int L, const FastDiv &U, int ug) {
   PrefillRange r;
-  r.units = qlen > 0 ? ((qlen + 31) >> 5) * G.d : 0;
+  r.units = qlen > 0 ? ((qlen + 31) >> 5) * U.d : 0;
   int u_last = 4 * ug + 3;
   u_last = u_last < r.units ? u_last : r.units - 1;
-  const int t_last = u_last >= 0 ? 32 * (u_last / G) : 0;
+  const int t_last = u_last >= 0 ? 32 * (u_last / U) : 0;
   const int last = (t_last + 32 < qlen ? t_last + 32 : qlen) - 1;
   r.kend = L - qlen + last + 1;
   r.n_steps = r.kend > 0 ? (r.kend + 63) >> 6 : 0;
@@ -187,7 +188,7 @@ __device__ __forceinline__ int prefill_prefix(int *pfx, int *red, const int32_t 
       const int qlen = cu_q[b + 1] - cu_q[b];
       int L = seq_lens[b];
       L = L < max_seq ? L : max_seq;
-      const PrefillRange r = prefill_range(qlen, L, pg.by_G, ug);
+      const PrefillRange r = prefill_range(qlen, L, pg.by_U, ug);
       if (4 * ug < r.units) c[k] = r.n_steps > 0 ? r.n_steps : 1;
     }
     sum += c[k];
@@ -341,7 +342,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
   const uint8_t *__restrict__ const kc = ap->kc, *__restrict__ const vc = ap->vc;
   const float *__restrict__ const ksc = ap->ksc, *__restrict__ const vsc = ap->vsc;
   const int32_t *__restrict__ const cu_q = ap->cu_q;
-  const FastDiv G = ap->pg.by_G;
+  const FastDiv U = ap->pg.by_U;
+  const int G = ap->pg.G;
   const int Hkv = ap->Hkv, BS = ap->BS, Mb = ap->Mb, nb = ap->nb;
   const float scale_log2 = ap->scale_log2;
   b = __builtin_amdgcn_readfirstlane(b);
@@ -351,7 +353,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
   int L = ap->seq_lens[b];
   const int qlen = q1 - q0;
   L = L < ap->max_seq ? L : ap->max_seq;
-  PrefillRange rg = prefill_range(qlen, L, G, ug);
+  PrefillRange rg = prefill_range(qlen, L, U, ug);
   rg.units = __builtin_amdgcn_readfirstlane(rg.units);
   rg.kend = __builtin_amdgcn_readfirstlane(rg.kend);
   rg.n_steps = __builtin_amdgcn_readfirstlane(rg.n_steps);
@@ -363,11 +365,12 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
     __syncthreads();  // the LDS of the unit group before (or of the prefix) is free
   }
   const bool partial = SHARED && take < all_steps;
-  const bool active = 4 * ug + wave < rg.units;  // an idle wave still copies its tile of every step
-  const int unit = active ? 4 * ug + wave : rg.units - 1;
-  const int qt = __builtin_amdgcn_readfirstlane(unit / G);
+  const int unit = 4 * ug + wave < rg.units ? 4 * ug + wave : rg.units - 1;
+  const int qt = __builtin_amdgcn_readfirstlane(unit / U);
   const int t0 = qt * 32;
-  const int h = kvh * G.d + (unit - qt * G.d);
+  // an idle wave (past the units, or a unit without a head) still copies its tile of every step
+  const bool active = 4 * ug + wave == unit && unit - qt * U.d < G;
+  const int h = kvh * G + (active ? unit - qt * U.d : 0);
   const int ctx = L - qlen;
   // Q^T operand j: lane l holds d = 16 j + 8 (l/32) .. + 7 of query t0 + l % 32.
   bf16x8 qb[D / 16];
@@ -825,8 +828,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_merge_kernel(
   const int lane = threadIdx.x & 63, n = lane & 31, hh = lane >> 5;
   const int q0 = cu_q[b];
   const int qlen = cu_q[b + 1] - q0;
-  const FastDiv G = pg.by_G;
-  const int units = qlen > 0 ? ((qlen + 31) >> 5) * G.d : 0;
+  const FastDiv U = pg.by_U;
+  const int units = qlen > 0 ? ((qlen + 31) >> 5) * U.d : 0;
   const int unit = 4 * ug + wave;
   const int n_e = __builtin_amdgcn_readfirstlane(pfx[e + 1] - pfx[e]);
   if (n_e <= 0 || unit >= units) return;
@@ -847,8 +850,9 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_merge_kernel(
   const float *p0 = part + ((2 * static_cast<int64_t>(w0) + (prefill_share(w0, T, W) < x0 ? 1 : 0)) * 4 + wave) * PF;
   const float *pn = part + (2 * static_cast<int64_t>(w0 + 1) * 4 + wave) * PF;  // the later parts, 8 PF apart
   const int np = w1 - w0;
-  const int qt = __builtin_amdgcn_readfirstlane(unit / G);
-  const int h = kvh * G.d + (unit - qt * G.d);
+  const int qt = __builtin_amdgcn_readfirstlane(unit / U);
+  if (unit - qt * U.d >= pg.G) return;  // a unit without a head
+  const int h = kvh * pg.G + (unit - qt * U.d);
   float M = p0[32 * D + n];
 #pragma unroll 4
   for (int s = 0; s < np; ++s) M = fmaxf(M, pn[s * (8 * PF) + 32 * D + n]);
@@ -888,7 +892,8 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
                                 int share, bool may_share) {
   PrefillGrid pg;
   const int64_t n_qt = (static_cast<int64_t>(max_query_len) + 31) / 32;
-  pg.n_ug = static_cast<int>((n_qt * G + 3) / 4);
+  int U = G;
+  pg.n_ug = static_cast<int>((n_qt * U + 3) / 4);
   pg.batch = batch;
   const int64_t items = static_cast<int64_t>(batch) * Hkv;
   const int64_t wgs = items * pg.n_ug;
@@ -924,6 +929,18 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
       }
     }
   }
+  // At most one unit group per CU with a tile's units to themselves (made up to
+  // a multiple of four by units without a head): so, as the chip has room for
+  // them and no group then runs on to a later tile's keys nor its waves on
+  // keys that they do not see. Past that, packed: the idle waves cost more.
+  // (us, packed -> not: one prompt of 512 at 16/8 heads bf16 20.9 -> 19.7, fp8
+  // 23.0 -> 21.1; at 28/4 21.3 -> 20.6; 256 groups so, two prompts of 512 at 16/8
+  // 22.2 -> 21.0; but 512 groups, four prompts, 25.2 -> 28.5.)
+  const int64_t tile_ug = (G + 3) / 4;
+  if (pg.W == 0 && items * n_qt * tile_ug <= kPrefillCus) {
+    U = static_cast<int>(4 * tile_ug);
+    pg.n_ug = static_cast<int>(n_qt * tile_ug);
+  }
   // Items are dealt to the eight XCDs in turn: R makes the KV heads of one
   // sequence (its unit groups dealt over R XCDs where there are fewer than
   // eight) cover all of them, so that sequences of different lengths load the
@@ -936,7 +953,8 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
   pg.n_sub = static_cast<int>(items * pg.R);
   pg.log2R = 0;
   while ((1 << pg.log2R) < pg.R) ++pg.log2R;
-  pg.by_G = fast_div(G);
+  pg.G = G;
+  pg.by_U = fast_div(U);
   pg.by_ug = fast_div(pg.n_ug);
   pg.by_inner = fast_div(pg.n_inner);
   pg.by_Hkv = fast_div(Hkv);
