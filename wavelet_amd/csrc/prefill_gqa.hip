@@ -273,7 +273,8 @@ __device__ __forceinline__ float load_scalar(const float *p) {
 }
 
 // SHARED: workgroups share the launch's steps evenly (PrefillGrid::W), else one per unit group.
-template <int D, bool FP8, bool SHARED>
+// SPAN: unit groups may span query tiles (PrefillGrid::by_U).
+template <int D, bool FP8, bool SHARED, bool SPAN>
 __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(PrefillArgs kernel_args) {
   using LT = LdsTile<D>;
   static_assert(kPrefillWaves == 4, "one tile per wave per 64-key step");
@@ -400,6 +401,10 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
   const int n_tiles = (kend + 15) / 16 < 4 * n_steps ? (kend + 15) / 16 : 4 * n_steps;
   const int region = D * BS * ESZ;
   const int min_pos = ctx + t0 - key0;  // the smallest query position of the wave
+  // One past the last key any query of this wave sees: below kend where the unit
+  // group goes on to later query tiles, whose keys must not reach this wave's
+  // products (a masked key's probability is 0, but 0 times a V that is not finite is NaN).
+  const int wend = min_pos + 32 < kend ? min_pos + 32 : kend;
 
   // Copy k of lane l moves piece p = 64 k + l of the wave's tile's K or V
   // (LDS offset 16 p). K piece p (both dtypes: 16-byte chunks): chunk p >> 4,
@@ -662,6 +667,27 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
       }
     }
   };
+  // The same with the keys at or past the wave's last left out: tiles skipped,
+  // the slots of its partial tile zeroed in the operand.
+  auto pv_end = [&](int s) {
+    const uint8_t *lv = ldsv + (s & 1) * 4 * VB + hh * D * 16 + n * 16;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int left = wend - 64 * s - 16 * t;  // keys of the tile that the wave sees
+      if (left <= 0) continue;                  // uniform
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, (u32x4{pw[t][0], pw[t][1], pw[t][2], pw[t][3]}));
+      u32x4 seen;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        seen[i] = (8 * hh + 2 * i < left ? 0xFFFFu : 0u) | (8 * hh + 2 * i + 1 < left ? 0xFFFF0000u : 0u);
+#pragma unroll
+      for (int c = 0; c < D / 32; ++c) {
+        const u32x4 w = *reinterpret_cast<const u32x4 *>(lv + t * VB + 32 * c * 16) & seen;
+        o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), pb, o[c], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
   // One step of the pipeline: finish step s (its scores in c0, c1 are
   // exponents against the reference) while scoring step s + 1 into n0, n1.
   auto body = [&](int s, floatx16 &c0, floatx16 &c1, floatx16 &n0, floatx16 &n1) {
@@ -736,15 +762,53 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
     };
     const int n_body = n_steps - 1;
     int s = 0;
-    for (; s + 2 <= n_body; s += 2) {
-      body(s, a0, a1, b0, b1);
-      body(s + 1, b0, b1, a0, a1);
-    }
-    if (s < n_body) {
-      body(s, a0, a1, b0, b1);
-      tail(s + 1, b0, b1);
+    if constexpr (!SPAN) {
+      for (; s + 2 <= n_body; s += 2) {
+        body(s, a0, a1, b0, b1);
+        body(s + 1, b0, b1, a0, a1);
+      }
+      if (s < n_body) {
+        body(s, a0, a1, b0, b1);
+        tail(s + 1, b0, b1);
+      } else {
+        tail(s, a0, a1);
+      }
     } else {
-      tail(s, a0, a1);
+      // A wave whose keys end before the steps do stops its products with the
+      // step that holds its last key; its copies go on as the others'.
+      const bool ends = wend < kend && wend < 64 * n_steps;  // uniform
+      const int n_whole = ends && wend < 64 * n_body ? (wend > 0 ? wend >> 6 : 0) : n_body;
+      for (; s + 2 <= n_whole; s += 2) {
+        body(s, a0, a1, b0, b1);
+        body(s + 1, b0, b1, a0, a1);
+      }
+      if (s < n_whole) {
+        body(s, a0, a1, b0, b1);
+        ++s;
+        a0 = b0;
+        a1 = b1;
+      }
+      if (!ends) {
+        tail(s, a0, a1);
+      } else {
+        const int s_last = s;
+        for (; s < n_steps; ++s) {
+          wait_vmcnt<0>();
+          if (s < n_body) {
+            land_body(s);
+            barrier_lds();
+            issue_v(s + 1, (s + 1) & 1);
+            issue_k(s + 2, s & 1);
+          } else {
+            land(s);
+            barrier_lds();
+          }
+          if (s == s_last) {
+            probs(a0, a1);
+            pv_end(s);
+          }
+        }
+      }
     }
   }
   if (active) {
@@ -1030,13 +1094,15 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
                          out_stride_h, cu_seqlens_q, seq_lens, block_table, bt_stride, max_blocks_per_seq, max_seq,
                          Hkv, BS, static_cast<int>(cache->num_blocks), scale_log2, fast_div(BS), pg,
                          static_cast<float *>(workspace), sinks};
-#define WKV_PREFILL_S(Dv, F8, SH) prefill_gqa_kernel<Dv, F8, SH><<<grid, 64 * kPrefillWaves, 0, s>>>(args)
-#define WKV_PREFILL(Dv, F8)         \
-  do {                              \
-    if (pg.W > 0)                   \
-      WKV_PREFILL_S(Dv, F8, true);  \
-    else                            \
-      WKV_PREFILL_S(Dv, F8, false); \
+  const bool span = pg.by_U.d % 4 != 0;
+#define WKV_PREFILL_S(Dv, F8, SH, SP) prefill_gqa_kernel<Dv, F8, SH, SP><<<grid, 64 * kPrefillWaves, 0, s>>>(args)
+#define WKV_PREFILL(Dv, F8)                                                         \
+  do {                                                                              \
+    if (pg.W > 0) {                                                                 \
+      if (span) WKV_PREFILL_S(Dv, F8, true, true); else WKV_PREFILL_S(Dv, F8, true, false);   \
+    } else {                                                                        \
+      if (span) WKV_PREFILL_S(Dv, F8, false, true); else WKV_PREFILL_S(Dv, F8, false, false); \
+    }                                                                               \
   } while (0)
   if (D == 128) {
     if (fp8) WKV_PREFILL(128, true); else WKV_PREFILL(128, false);
