@@ -1,13 +1,17 @@
-"""Prefill launch grids: how query heads and tiles are packed into workgroups, by the sizes.
-Against the float64 oracle."""
+"""Prefill launch grids: how query heads and tiles are packed into workgroups, and when a launch
+shares its keys, by the sizes and length bounds the caller gives. Against the float64 oracle."""
 
+import numpy as np
 import pytest
 import torch
 
-from kvcase import to_dev_bits
+from kvcase import bits_of, check_attention, to_dev_bits
+from oracle import fp8, paged
 from test_gpu_prefill import BF16, _case, _run_and_check
-from test_gpu_prefill_shared import _shared_call
-from wavelet_amd import prefill_gqa
+from test_gpu_prefill_shared import _reference, _shared_call
+from wavelet_amd import _lib, prefill_gqa
+from wavelet_amd.cache import KV_DTYPES
+from wavelet_amd.plan import PrefillStep
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +57,87 @@ def test_values_of_later_tiles_that_are_not_finite(cuda, hq, hkv, d, n_seq, shar
     clean, got = outs
     assert torch.isfinite(clean).all() and torch.isnan(got[161:270]).all()
     assert torch.equal(got[:160], clean[:160]) and torch.equal(got[270:], clean[270:])
+
+
+def _need(w, cache, cu, keys):
+    return _lib.load().wkv_prefill_workspace_size(w.batch, KV_DTYPES[cache.kv_dtype], w.num_kv_heads, w.num_q_heads,
+                                                  w.head_dim, int(np.diff(cu).max()), keys, 0)
+
+
+@pytest.mark.parametrize("sinks", [False, True])
+@pytest.mark.parametrize("kv_dtype", ["bf16", "fp8_e4m3"])
+@pytest.mark.parametrize("hq,hkv,d,qlens,lens", [(28, 4, 128, [1, 1, 1], [5000, 4096, 3000]),
+                                                 (14, 2, 64, [70, 33, 1], [4000, 700, 2049]),
+                                                 (32, 8, 128, [40, 0], [3000, 64])])
+def test_launches_shared_by_the_librarys_choice(cuda, hq, hkv, d, qlens, lens, kv_dtype, sinks):
+    w, cache, host, new = _case(cuda, f"pfauto{hq}{d}", hq, hkv, d, 16, qlens, lens, kv_dtype)
+    assert _need(w, cache, new[4], max(lens)) > 0
+    if not sinks:
+        _run_and_check(cuda, w, cache, host, new, f"auto {hq}/{hkv}")
+        return
+    s = np.linspace(-2, 12, hq).astype(np.float32)
+    kn, vn, q, nslots, cu = new
+    out = prefill_gqa(to_dev_bits(q, BF16, cuda), cache, torch.from_numpy(w.block_tables).to(cuda),
+                      torch.from_numpy(w.context_lens).to(cuda), torch.from_numpy(cu).to(cuda), w.scale,
+                      key=to_dev_bits(kn, BF16, cuda), value=to_dev_bits(vn, BF16, cuda),
+                      slot_mapping=torch.from_numpy(nslots).to(cuda), sinks=torch.from_numpy(s).to(cuda))
+    ref = _reference(w, cache, host, new, s)
+    plain = paged.prefill_gqa(paged.bf16_to_f32(q), *_logical(host), w.block_tables, w.context_lens, cu, w.scale)
+    # (over thousands of keys the outputs are small: what the sinks change is a part of them, ten
+    # times the relative tolerance or more)
+    assert np.linalg.norm(ref - plain) > 0.1 * np.linalg.norm(plain)
+    check_attention(paged.bf16_to_f32(bits_of(out)), ref, f"auto sinks {hq}/{hkv}")
+
+
+def _logical(host):
+    kc, vc, ks, vs = host
+    if ks is None:
+        return tuple(paged.bf16_to_f32(x) for x in paged.logical_kv(kc, vc))
+    shape = (len(ks), kc.shape[3], kc.shape[1], kc.shape[2] * kc.shape[4])
+    return (fp8.dequantize(paged.k_logical(kc).reshape(shape), ks[:, None, :, None]),
+            fp8.dequantize(paged.v_logical(vc), vs[:, None, :, None]))
+
+
+@pytest.mark.parametrize("kv_dtype", ["bf16", "fp8_e4m3"])
+def test_layers_of_a_plan_take_turns_with_its_workspace(cuda, kv_dtype):
+    """Three layers of different contents (and of two head layouts) over one plan, shared by the library's
+    choice, run twice."""
+    qlens, lens = [3, 50, 1], [4000, 2500, 3000]
+    layers = [_case(cuda, "pfplan", hq, hkv, 128, 16, qlens, lens, kv_dtype) for hq, hkv in [(28, 4), (16, 4), (28, 4)]]
+    wl, cache, host, (kn, vn, q, nslots, cu) = layers[2]
+    layers[2] = wl, cache, host, (vn, kn, q ^ np.uint16(0x8000), nslots, cu)
+    w, _, _, (_, _, _, nslots, cu) = layers[0]
+    dev = [[to_dev_bits(new[i], BF16, cuda) for _, _, _, new in layers] for i in (2, 0, 1)]  # q, key, value
+    outs = [torch.full_like(q, float("nan")) for q in dev[0]]
+    assert all(_need(x[0], x[1], cu, max(lens)) > 0 for x in layers)
+    assert all(np.array_equal(x[0].block_tables, w.block_tables) for x in layers)
+    step = PrefillStep([x[1] for x in layers], dev[0], dev[1], dev[2], outs, torch.from_numpy(w.block_tables).to(cuda),
+                       torch.from_numpy(w.context_lens).to(cuda), torch.from_numpy(cu).to(cuda),
+                       torch.from_numpy(nslots).to(cuda), w.scale, max(qlens), max(lens))
+    for _ in range(2):
+        step.run()
+    for i, (wl, cache, host, new) in enumerate(layers):
+        check_attention(paged.bf16_to_f32(bits_of(outs[i])), _reference(wl, cache, host, new), f"layer {i}")
+
+
+@pytest.mark.parametrize("kv_dtype", ["bf16", "fp8_e4m3"])
+@pytest.mark.parametrize("hq,hkv,d,qlens,lens", [(32, 8, 128, [200], [200]), (14, 2, 64, [60, 1, 0, 33], [260, 3, 40, 33]),
+                                                 (28, 4, 128, [37, 250, 1], [37, 250, 900]),
+                                                 (28, 4, 128, [16, 1], [6000, 300]), (16, 8, 128, [0, 1], [5, 70])])
+def test_length_bounds_above_the_lengths(cuda, hq, hkv, d, qlens, lens, kv_dtype):
+    """A caller that gives the model's limit for max_seq_len gets a launch that could share; what it does
+    follows the lengths on the device. Where that is whole unit groups, the bits are the plain launch's."""
+    w, cache, host, new = _case(cuda, f"pfbound{hq}{len(qlens)}", hq, hkv, d, 16, qlens, lens, kv_dtype)
+    kn, vn, q, nslots, cu = new
+    bt = torch.full((w.batch, 16384 // 16), -1, dtype=torch.int32, device=cuda)
+    bt[:, :w.block_tables.shape[1]] = torch.from_numpy(w.block_tables).to(cuda)
+    args = (to_dev_bits(q, BF16, cuda), cache, bt, torch.from_numpy(w.context_lens).to(cuda),
+            torch.from_numpy(cu).to(cuda), w.scale)
+    assert _need(w, cache, cu, 16384) > 0
+    cache.append(to_dev_bits(kn, BF16, cuda), to_dev_bits(vn, BF16, cuda), torch.from_numpy(nslots).to(cuda))
+    mql = max(qlens)
+    out = torch.full((len(q), hq, d), float("nan"), dtype=BF16, device=cuda)
+    prefill_gqa(*args, max_query_len=mql, max_seq_len=16384, out=out)
+    check_attention(paged.bf16_to_f32(bits_of(out)), _reference(w, cache, host, new), "bounds")
+    if max(lens) <= 300:
+        assert torch.equal(out, prefill_gqa(*args, max_query_len=mql, max_seq_len=max(lens)))

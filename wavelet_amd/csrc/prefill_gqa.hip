@@ -23,10 +23,10 @@
 // 32x32x16 bf16 MFMAs. fp8 tiles are dequantized in LDS (exactly:
 // power-of-two scales) by the wave that copied them, so both dtypes share the
 // attention arithmetic. Tiles on the causal diagonal mask per lane (column).
-// A grid too small for the chip (a few new tokens over a long context) shares
-// its 64-key steps evenly over a fixed number of workgroups instead
-// (prefill_grid): a workgroup's share may end inside a unit group, whose parts
-// leave fp32 partials that prefill_merge_kernel combines by log-sum-exp.
+// A grid too small for the chip (a few new tokens over a long context) may share
+// its 64-key steps evenly over a number of workgroups instead (share_workgroups):
+// a workgroup's share may end inside a unit group, whose parts leave fp32
+// partials that prefill_merge_kernel combines by log-sum-exp.
 #include "gqa_tiles.h"
 #include "lds_dma.h"
 
@@ -35,18 +35,58 @@
 namespace wkv {
 
 constexpr int kPrefillWaves = 4;
-// The rule that shares a launch's steps over a fixed number of workgroups
-// (prefill_grid) compares two estimates in microseconds, fitted to launches of
-// 16 to 376 unit groups over 500 to 15,000 keys (bf16, d=128):
 constexpr int kPrefillCus = 256;
-constexpr int kShareMinKeys = 1024;   // below, no estimate favours sharing (its second launch alone costs the gain)
-constexpr double kStepUs = 1.08;      // one 64-key step of a workgroup alone on its CU, bf16
-constexpr double kStepFp8Us = 1.45;   // ... fp8 (the conversion stands before the barrier)
-constexpr double kStepPairUs = 2.0;   // a step of each of two on a CU, either type
-constexpr double kPartUs = 0.05;      // writing and merging a workgroup's partials
-constexpr double kGroupUs = 6.0;      // starting a unit group (its queries, table and first keys)
-constexpr double kLaunchUs = 5.0;     // a plain launch's fixed part
-constexpr double kShareUs = 9.5;      // a shared launch's: with the prefix and the merge's launch
+constexpr int kShareMinKeys = 1024;  // below, no estimate favours sharing (its second launch alone costs the gain)
+
+// The rule that shares a launch's steps over a number of workgroups compares
+// estimates in microseconds, fitted to launches of 8 to 1,000 unit groups over
+// 400 to 17,000 keys.
+struct ShareCost {
+  float alone;  // one 64-key step of a workgroup alone on its CU
+  float pair;   // ... of each of two on a CU
+  float tail;   // the last workgroups of more than one per CU, as a share of the longest chain
+  float gain;   // shared where the estimate is below this share of the plain launch's
+};
+template <int D, bool FP8>
+__host__ __device__ constexpr ShareCost share_cost() {
+  return FP8 && D == 64 ? ShareCost{1.2f, 1.5f, 0.1f, 0.85f} : ShareCost{FP8 ? 1.45f : 1.08f, 2.0f, 0.3f, 0.75f};
+}
+constexpr float kPartUs = 0.05f;   // writing and merging a workgroup's partials
+constexpr float kGroupUs = 6.0f;   // starting a unit group (its queries, table and first keys)
+constexpr float kLaunchUs = 5.0f;  // a plain launch's fixed part
+constexpr float kShareUs = 9.5f;   // a shared launch's: with the prefix and the merge's launch
+
+// Workgroups (a multiple of 64, at most `most`) that are expected to share T
+// steps of `groups` unit groups, the longest of `longest` steps, faster than a
+// workgroup per group would take them; 0: none. PAID: the shared launch's fixed
+// part is spent either way.
+// Measured (us, plain -> shared): 4 x 37-250 new tokens over 5-15K keys at
+// 28/4 heads 241 -> 131 (fp8 352 -> 131), 64 over 2K at 32/8 38 -> 23,
+// 8 x 20-60 over 4-12K at 32/4 fp8 275 -> 82, 1,000 over 8K at 16/8 147 ->
+// 87; but 16 x 16 over 1K 22.5 -> 27.3, one prompt of 1,500 tokens 36 -> 55
+// and of 512 15 -> 29, two of 2,048 at 14/2 fp8 41 -> 62: short chains gain less
+// than the partials and the second launch cost. Over 2,172 shapes (those heads,
+// 1-16 sequences, 1-2,048 new tokens over 0-15K) the choice is at worst 11%
+// slower than the plain launch (3 by more than 5%) and 4% from the best of both.
+template <int D, bool FP8, bool PAID>
+__host__ __device__ __forceinline__ int share_workgroups(float T, float longest, float groups, int most) {
+  constexpr ShareCost c = share_cost<D, FP8>();
+  float best = longest * c.alone;
+  if (groups > kPrefillCus) best = fmaxf(best, T / (2 * kPrefillCus) * c.pair) + c.tail * longest * c.alone;
+  best = PAID ? best + kShareUs : (best + kLaunchUs) * c.gain;
+  int W = 0;
+#pragma unroll
+  for (int w = 64; w <= 2 * kPrefillCus; w += 64) {
+    const bool two = w > kPrefillCus;
+    const float us = T * ((two ? c.pair : c.alone) / w) + kPartUs * w * D / 128 +
+                     (two ? 0.5f : 1.f) * kGroupUs * (1.f + groups * (1.f / w)) + kShareUs;
+    if (w <= most && us < best) {
+      best = us;
+      W = w;
+    }
+  }
+  return W;
+}
 
 // Eight e4m3fn codes (bytes of lo, then hi) times a power-of-two scale as
 // eight bf16 values, by the hardware pair conversion (exact: every such
@@ -137,7 +177,8 @@ struct PrefillGrid {
   int R;        // XCDs the unit groups of one (sequence, KV head) are dealt over
   int n_inner;  // workgroups of one (sequence, KV head) per XCD
   int n_sub;    // (sequence, KV head) x R
-  int W;        // workgroups that share the steps evenly; 0: a workgroup per unit group
+  int W;        // most workgroups that share the steps evenly (share_workgroups); 0: a workgroup per unit group
+  int forced;   // the caller's number of them: W whatever the lengths
   int batch;
   int log2R;
   int G;                                  // query heads per KV head
@@ -170,15 +211,25 @@ __device__ __forceinline__ PrefillRange prefill_range(int qlen, int L, const Fas
 // mix of lengths, and at most its first and last unit groups are partial.
 // pfx[i] (LDS) is the line's prefix at entry i = sequence * n_ug + group of
 // one KV head, entries in order, pfx[E] their total; every workgroup forms it
-// itself from the lengths (a launch of its own would cost more).
+// itself from the lengths (a launch of its own would cost more). The host knows
+// bounds of the lengths only: the number of workgroups is chosen here again from
+// the lengths themselves, and where sharing does not pay a workgroup takes a
+// whole unit group (with bounds of 16,384 keys over prompts of 200 at 32/8 heads, for
+// one, that is the plain launch's work with the prefix and an empty merge).
 constexpr int kPrefillEntries = 1024;  // at most this many entries per KV head
 
-__device__ __forceinline__ int prefill_prefix(int *pfx, int *red, const int32_t *cu_q, const int32_t *seq_lens,
-                                              int max_seq, const PrefillGrid &pg) {
+struct PrefillLine {
+  int total, longest, groups;  // of one KV head: steps, steps of the longest unit group, unit groups with queries
+};
+
+template <bool STATS>  // else the total alone
+__device__ __forceinline__ PrefillLine prefill_prefix(int *pfx, int *red, const int32_t *cu_q,
+                                                      const int32_t *seq_lens, int max_seq,
+                                                      const PrefillGrid &pg) {
   const int E = pg.batch * pg.n_ug;
   const int per = (E + 64 * kPrefillWaves - 1) / (64 * kPrefillWaves);  // <= 4 entries per thread
   const int e0 = threadIdx.x * per;
-  int c[kPrefillEntries / (64 * kPrefillWaves)], sum = 0;
+  int c[kPrefillEntries / (64 * kPrefillWaves)], sum = 0, mx = 0, n = 0;
 #pragma unroll
   for (int k = 0; k < kPrefillEntries / (64 * kPrefillWaves); ++k) {
     c[k] = 0;
@@ -192,6 +243,8 @@ __device__ __forceinline__ int prefill_prefix(int *pfx, int *red, const int32_t 
       if (4 * ug < r.units) c[k] = r.n_steps > 0 ? r.n_steps : 1;
     }
     sum += c[k];
+    mx = c[k] > mx ? c[k] : mx;
+    n += __popcll(__ballot(c[k] > 0));  // of the wave
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int incl = sum;
@@ -200,13 +253,23 @@ __device__ __forceinline__ int prefill_prefix(int *pfx, int *red, const int32_t 
     const int y = __shfl_up(incl, o, 64);
     if (lane >= o) incl += y;
   }
-  if (lane == 63) red[wave] = incl;
+  if constexpr (STATS) mx = wave_reduce(mx, [](int a, int b) { return a > b ? a : b; });
+  if (lane == 63) {
+    red[wave] = incl;
+    red[kPrefillWaves + wave] = mx;
+    red[2 * kPrefillWaves + wave] = n;
+  }
   __syncthreads();
-  int base = incl - sum, total = 0;
+  int base = incl - sum;
+  PrefillLine line{0, 0, 0};
 #pragma unroll
   for (int w = 0; w < kPrefillWaves; ++w) {
     if (w < wave) base += red[w];
-    total += red[w];
+    line.total += red[w];
+    if constexpr (STATS) {
+      line.longest = red[kPrefillWaves + w] > line.longest ? red[kPrefillWaves + w] : line.longest;
+      line.groups += red[2 * kPrefillWaves + w];
+    }
   }
 #pragma unroll
   for (int k = 0; k < kPrefillEntries / (64 * kPrefillWaves); ++k)
@@ -214,9 +277,10 @@ __device__ __forceinline__ int prefill_prefix(int *pfx, int *red, const int32_t 
       pfx[e0 + k] = base;
       base += c[k];
     }
-  if (threadIdx.x == 0) pfx[E] = total;
+  if (threadIdx.x == 0) pfx[E] = line.total;
   __syncthreads();
-  return __builtin_amdgcn_readfirstlane(total);
+  return PrefillLine{__builtin_amdgcn_readfirstlane(line.total), __builtin_amdgcn_readfirstlane(line.longest),
+                     __builtin_amdgcn_readfirstlane(line.groups)};
 }
 
 // First step of workgroup w's share of T steps over W workgroups (the callers
@@ -228,10 +292,16 @@ __device__ __forceinline__ int64_t prefill_share(int w, int64_t T, int W) { retu
 // output accumulators as the lanes hold them, so both the store and the
 // merge's load are whole 1 KB wave accesses), then the 32 queries' reference
 // maxima (log2 domain) and sums. Workgroup w owns partial slots 2 w (its first
-// unit group) and 2 w + 1 (a later one), four units each.
+// unit group) and 2 w + 1 (a later one), four units each. Behind the slots of
+// the grid's W workgroups: the number that did share (an int), for the merge.
 template <int D>
 constexpr int prefill_part_floats() {
   return 32 * D + 64;
+}
+constexpr int kShareTailBytes = 16;
+template <int D>
+__device__ __forceinline__ int *prefill_shared_by(float *part, int W) {
+  return reinterpret_cast<int *>(part + static_cast<int64_t>(W) * 2 * 4 * prefill_part_floats<D>());
 }
 
 // The attention kernel's arguments: one struct, the kernel's only parameter
@@ -297,33 +367,54 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
   // first load of the queries).
   // (not volatile: that would count as a write, and loads after it as vector loads)
   asm("" : "+s"(id) : "s"(kernel_args.kc), "s"(kernel_args.o_sh), "s"(kernel_args.pg.n_ug), "s"(kernel_args.sinks));
-  int b, kvh, ug, s_begin = 0, seg = 0;
+  int b, kvh, ug, s_begin = 0;
+  int part_slot = 0;       // SHARED: this workgroup's partial slot of the unit group (odd past its first)
   int64_t steps_left = 0;  // SHARED: of this workgroup's share
   if constexpr (SHARED) {
     const PrefillArgs &a = prefill_args();
     const PrefillGrid pg = a.pg;
-    // XCD i mod 8 takes a contiguous eighth of the line: its workgroups read the same keys.
-    const int w = (id & 7) * (pg.W / 8) + id / 8;
     int *pfx = reinterpret_cast<int *>(ldsk);
-    static_assert((kPrefillEntries + 1 + kPrefillWaves) * 4 <= 2 * 4 * KB, "the prefix fits the K slots");
+    static_assert((kPrefillEntries + 1 + 3 * kPrefillWaves) * 4 <= 2 * 4 * KB, "the prefix fits the K slots");
     const int E = pg.batch * pg.n_ug;
-    const int total = prefill_prefix(pfx, pfx + kPrefillEntries + 1, a.cu_q, a.seq_lens, a.max_seq, pg);
+    const PrefillLine line = prefill_prefix<true>(pfx, pfx + kPrefillEntries + 1, a.cu_q, a.seq_lens, a.max_seq, pg);
+    const int total = line.total;
     const int64_t T = static_cast<int64_t>(total) * a.Hkv;
-    const int W = T < pg.W ? static_cast<int>(T) : pg.W;
-    if (w >= W) return;
-    const int64_t x0 = prefill_share(w, T, W);
-    steps_left = prefill_share(w + 1, T, W) - x0;
-    kvh = static_cast<int>(x0 / total);
-    const int y = static_cast<int>(x0 - static_cast<int64_t>(kvh) * total);
-    int lo = 0, hi = E;  // the last entry with pfx <= y (entries of no steps share their successor's prefix)
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (pfx[mid] <= y) lo = mid; else hi = mid;
+    int W = pg.W;
+    if (!pg.forced)
+      W = share_workgroups<D, FP8, true>(static_cast<float>(T), static_cast<float>(line.longest),
+                                         static_cast<float>(line.groups) * static_cast<float>(a.Hkv), pg.W);
+    W = __builtin_amdgcn_readfirstlane(W);
+    if (id == 0 && threadIdx.x == 0) *prefill_shared_by<D>(a.part, pg.W) = W;
+    int e;
+    if (W > 0) {
+      // XCD i mod 8 takes a contiguous eighth of the line: its workgroups read the same keys.
+      if (id >= W) return;
+      const int w = (id & 7) * (W / 8) + id / 8;
+      W = T < W ? static_cast<int>(T) : W;
+      if (w >= W) return;
+      const int64_t x0 = prefill_share(w, T, W);
+      steps_left = prefill_share(w + 1, T, W) - x0;
+      kvh = static_cast<int>(x0 / total);
+      const int y = static_cast<int>(x0 - static_cast<int64_t>(kvh) * total);
+      int lo = 0, hi = E;  // the last entry with pfx <= y (entries of no steps share their successor's prefix)
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (pfx[mid] <= y) lo = mid; else hi = mid;
+      }
+      e = __builtin_amdgcn_readfirstlane(lo);
+      s_begin = __builtin_amdgcn_readfirstlane(y - pfx[e]);
+      part_slot = 2 * w;
+    } else {
+      // A whole unit group each, the latest query tiles first.
+      const int n = E * a.Hkv, g = (id & 7) * ((n + 7) / 8) + id / 8;
+      if (id / 8 >= (n + 7) / 8 || g >= n) return;
+      kvh = g / E;
+      e = E - 1 - (g - kvh * E);
+      steps_left = __builtin_amdgcn_readfirstlane(pfx[e + 1] - pfx[e]);
+      if (steps_left <= 0) return;
     }
-    lo = __builtin_amdgcn_readfirstlane(lo);
-    s_begin = __builtin_amdgcn_readfirstlane(y - pfx[lo]);
-    b = lo / pg.by_ug;
-    ug = lo - b * pg.n_ug;
+    b = e / pg.by_ug;
+    ug = e - b * pg.n_ug;
   } else {
     const PrefillGrid &pg = kernel_args.pg;
     // Eight sub-items (item, share r of its unit groups) run at a time, one per XCD.
@@ -820,8 +911,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
     l = __uint_as_float(x[0]) + __uint_as_float(x[1]);
   }
   if (partial) {  // uniform
-    const int w = (id & 7) * (ae->pg.W / 8) + id / 8;
-    float *pp = ae->part + ((2 * static_cast<int64_t>(w) + (seg > 0 ? 1 : 0)) * 4 + wave) * prefill_part_floats<D>();
+    float *pp = ae->part + (static_cast<int64_t>(part_slot) * 4 + wave) * prefill_part_floats<D>();
 #pragma unroll
     for (int c = 0; c < D / 32; ++c)
 #pragma unroll
@@ -852,7 +942,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
   }
   if constexpr (SHARED) {
     steps_left -= take;
-    ++seg;
+    part_slot |= 1;
   }
   }
   if constexpr (!SHARED) break;
@@ -875,13 +965,16 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
 // there. Bound by reading the partials (66 KB per part at d=128).
 template <int D>
 __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_merge_kernel(
-    const float *__restrict__ part, uint16_t *__restrict__ out, int64_t o_st, int64_t o_sh,
+    float *__restrict__ part, uint16_t *__restrict__ out, int64_t o_st, int64_t o_sh,
     const int32_t *__restrict__ cu_q, const int32_t *__restrict__ seq_lens, int max_seq, int Hkv, PrefillGrid pg,
     const float *__restrict__ sinks) {
   constexpr int PF = prefill_part_floats<D>();
   __shared__ int pfx[kPrefillEntries + 1];
-  __shared__ int red[kPrefillWaves];
-  const int total = prefill_prefix(pfx, red, cu_q, seq_lens, max_seq, pg);
+  __shared__ int red[3 * kPrefillWaves];
+  const int by = *prefill_shared_by<D>(part, pg.W);  // (on its way while the prefix is formed)
+  const int total = prefill_prefix<false>(pfx, red, cu_q, seq_lens, max_seq, pg).total;
+  const int shared_by = __builtin_amdgcn_readfirstlane(by);
+  if (shared_by == 0) return;  // every unit group was taken whole
   const int E = pg.batch * pg.n_ug;
   const int kvh = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x / E));
   const int e = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x - kvh * E));
@@ -899,7 +992,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_merge_kernel(
   if (n_e <= 0 || unit >= units) return;
   // The workgroups whose shares [share(w), share(w + 1)) meet this group's steps [x0, x0 + n_e).
   const int64_t T = static_cast<int64_t>(total) * Hkv;
-  const int W = T < pg.W ? static_cast<int>(T) : pg.W;
+  const int W = T < shared_by ? static_cast<int>(T) : shared_by;
   const int64_t x0 = static_cast<int64_t>(kvh) * total + __builtin_amdgcn_readfirstlane(pfx[e]);
   const int64_t x1 = x0 + n_e;
   int w0 = static_cast<int>(x0 * W / T);
@@ -950,8 +1043,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_merge_kernel(
   }
 }
 
-// The launch's grid. With a workspace (may_share), the steps are shared over
-// W workgroups where that is expected to be faster; share > 0 sets W.
+// The launch's grid. With a workspace (may_share), the steps may be shared over
+// up to W workgroups where that is expected to be faster; share > 0 sets W.
 static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int max_query_len, int max_seq,
                                 int share, bool may_share) {
   PrefillGrid pg;
@@ -962,35 +1055,19 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
   const int64_t items = static_cast<int64_t>(batch) * Hkv;
   const int64_t wgs = items * pg.n_ug;
   pg.W = 0;
+  pg.forced = share > 0;
   if (may_share && static_cast<int64_t>(batch) * pg.n_ug <= kPrefillEntries) {
     if (share > 0) {
       pg.W = (share + 7) / 8 * 8;
     } else if (wgs < 4 * kPrefillCus && max_seq > kShareMinKeys) {
-      // Measured (us, plain -> shared): 4 x 37-250 new tokens over 5-15K keys at
-      // 28/4 heads 241 -> 131 (fp8 352 -> 131), 64 over 2K at 32/8 38 -> 23,
-      // 8 x 20-60 over 4-12K at 32/4 fp8 275 -> 82, 1,000 over 8K at 16/8 147 ->
-      // 87; but 16 x 16 over 1K 22.5 -> 27.3, one prompt of 1,500 tokens 36 -> 55
-      // and of 512 15 -> 29: short chains gain less than the partials and the
-      // second launch cost.
-      const double steps = max_seq > 64 ? max_seq / 64.0 : 1.0;
-      const double qsteps = max_query_len < max_seq ? max_query_len / 64.0 : steps;
+      const float steps = static_cast<float>(max_seq) / 64.f;
+      const float qsteps = max_query_len < max_seq ? static_cast<float>(max_query_len) / 64.f : steps;
       // the host knows the longest lengths only: several sequences are taken
       // to bring 0.6 of the longest one's work on average
-      const double T = wgs * (steps - 0.5 * qsteps) * (batch > 1 ? 0.6 : 1.0);
-      // plain: the longest chain or the chip's throughput, and a tail
-      const double alone = fp8 ? kStepFp8Us : kStepUs;
-      const double full = T / (2 * kPrefillCus) * kStepPairUs;
-      double best = fmax(steps * alone, full) + (wgs > kPrefillCus ? 0.3 * steps * alone : 0.0) + kLaunchUs;
-      best *= 0.75;  // shared only for a clear gain
-      for (int W = 64; W <= 2 * kPrefillCus; W += 64) {
-        const bool pair = W > kPrefillCus;
-        const double ts = T / W * (pair ? kStepPairUs : alone) + kPartUs * W * D / 128 +
-                          (pair ? 0.5 : 1.0) * kGroupUs * (1.0 + static_cast<double>(wgs) / W) + kShareUs;
-        if (ts < best) {
-          best = ts;
-          pg.W = W;
-        }
-      }
+      const float T = static_cast<float>(wgs) * (steps - 0.5f * qsteps) * (batch > 1 ? 0.6f : 1.f);
+      const auto choose = D == 128 ? (fp8 ? share_workgroups<128, true, false> : share_workgroups<128, false, false>)
+                                   : (fp8 ? share_workgroups<64, true, false> : share_workgroups<64, false, false>);
+      pg.W = choose(T, steps, static_cast<float>(wgs), 2 * kPrefillCus);
     }
   }
   // At most one unit group per CU with a tile's units to themselves (made up to
@@ -1026,7 +1103,7 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
 }
 
 static int64_t prefill_workspace(const PrefillGrid &pg, int D) {
-  return static_cast<int64_t>(pg.W) * 2 * 4 * (32 * D + 64) * 4;
+  return pg.W > 0 ? static_cast<int64_t>(pg.W) * 2 * 4 * (32 * D + 64) * 4 + kShareTailBytes : 0;
 }
 
 }  // namespace wkv
@@ -1081,7 +1158,11 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
   if (need > 0)
     WKV_CHECK_ARG(aligned16(workspace) && workspace_bytes >= need, "workspace too small: need %lld bytes, got %lld",
                   (long long)need, (long long)workspace_bytes);
-  const int64_t n_wg = pg.W > 0 ? pg.W : (static_cast<int64_t>(pg.n_sub) + 7) / 8 * 8 * pg.n_inner;
+  int64_t n_wg = (static_cast<int64_t>(pg.n_sub) + 7) / 8 * 8 * pg.n_inner;
+  if (pg.W > 0) {  // (unless forced, room for a workgroup per unit group: at most 1,024 of them)
+    const int64_t whole = pg.forced ? 0 : (static_cast<int64_t>(batch) * Hkv * pg.n_ug + 7) / 8 * 8;
+    n_wg = whole > pg.W ? whole : pg.W;
+  }
   WKV_CHECK_ARG(n_wg <= INT32_MAX, "prefill grid too large");
   const dim3 grid(static_cast<unsigned>(n_wg));
   auto s = static_cast<hipStream_t>(stream);
@@ -1115,11 +1196,11 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
   if (pg.W > 0) {
     const dim3 mgrid(static_cast<unsigned>(Hkv * batch * pg.n_ug), static_cast<unsigned>(D / 32));
     if (D == 128)
-      prefill_merge_kernel<128><<<mgrid, 64 * kPrefillWaves, 0, s>>>(static_cast<const float *>(workspace), oo,
+      prefill_merge_kernel<128><<<mgrid, 64 * kPrefillWaves, 0, s>>>(static_cast<float *>(workspace), oo,
                                                                      out_stride_t, out_stride_h, cu_seqlens_q, seq_lens,
                                                                      max_seq, Hkv, pg, sinks);
     else
-      prefill_merge_kernel<64><<<mgrid, 64 * kPrefillWaves, 0, s>>>(static_cast<const float *>(workspace), oo,
+      prefill_merge_kernel<64><<<mgrid, 64 * kPrefillWaves, 0, s>>>(static_cast<float *>(workspace), oo,
                                                                     out_stride_t, out_stride_h, cu_seqlens_q, seq_lens,
                                                                     max_seq, Hkv, pg, sinks);
     WKV_CHECK_LAUNCH("paged prefill merge");
