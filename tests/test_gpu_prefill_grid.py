@@ -23,6 +23,8 @@ pytestmark = pytest.mark.gpu
     (16, 8, 128, [256, 1, 90, 17], 48),
     (16, 8, 128, [257, 1, 90, 17], 48),
     (5, 1, 128, [289, 0, 128, 7] * 4, 20),
+    (8, 2, 64, [300, 1, 100, 60, 290, 33, 7, 256] * 4, 0),  # 768 workgroups: an XCD's sub-items in turn
+    (8, 2, 64, [400, 1, 100, 60, 290, 33, 7, 256] * 4, 0),  # 1,024: one after another
 ])
 def test_both_sides_of_the_packing_bounds(cuda, hq, hkv, d, qlens, ctx, kv_dtype):
     w, cache, host, new = _case(cuda, f"pfgrid{hq}{d}{max(qlens)}", hq, hkv, d, 16, qlens, [n + ctx + 1 for n in qlens],

@@ -176,6 +176,7 @@ struct PrefillGrid {
   int n_ug;     // unit groups (four units) per (sequence, KV head), at the longest query
   int R;        // XCDs the unit groups of one (sequence, KV head) are dealt over
   int n_inner;  // workgroups of one (sequence, KV head) per XCD
+  int mixed;    // an XCD takes its sub-items' workgroups in turn (by_inner: its sub-items), else one sub-item's after another's
   int n_sub;    // (sequence, KV head) x R
   int W;        // most workgroups that share the steps evenly (share_workgroups); 0: a workgroup per unit group
   int forced;   // the caller's number of them: W whatever the lengths
@@ -418,8 +419,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
   } else {
     const PrefillGrid &pg = kernel_args.pg;
     // Eight sub-items (item, share r of its unit groups) run at a time, one per XCD.
-    const int oct = (id >> 3) / pg.by_inner;
-    const int inner = (id >> 3) - oct * pg.n_inner;
+    const int q = (id >> 3) / pg.by_inner, r = (id >> 3) - q * pg.by_inner.d;
+    const int oct = pg.mixed ? r : q, inner = pg.mixed ? q : r;
     const int sub = 8 * oct + (id & 7);
     if (sub >= pg.n_sub) return;
     const int item = sub >> pg.log2R;
@@ -1097,7 +1098,15 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
   pg.G = G;
   pg.by_U = fast_div(U);
   pg.by_ug = fast_div(pg.n_ug);
-  pg.by_inner = fast_div(pg.n_inner);
+  // Up to three workgroups per CU, an XCD takes its sub-items in turn, the
+  // longest chains of all of them first; past that one sub-item after another,
+  // as their keys no longer stay in its L2 together. (us, after another -> in
+  // turn: two prompts of 2,048 at 14/2 heads 42.4 -> 38.0, four of 1,500 48.8 ->
+  // 41.1, two of 1,000 at 32/8 42.7 -> 39.2; but 1,024 workgroups, 16 of 256,
+  // 38.8 -> 53.4.)
+  const int n_oct = (pg.n_sub + 7) / 8;
+  pg.mixed = n_oct > 1 && static_cast<int64_t>(8) * n_oct * pg.n_inner <= 3 * kPrefillCus;
+  pg.by_inner = fast_div(pg.mixed ? n_oct : pg.n_inner);
   pg.by_Hkv = fast_div(Hkv);
   return pg;
 }
