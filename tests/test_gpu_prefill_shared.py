@@ -42,8 +42,11 @@ def _shared_call(cuda, w, cache, new, workgroups, sinks=None):
             bt.shape[1], w.batch, mql, msl, float(w.scale), workgroups]
     stream = torch.cuda.current_stream(cuda).cuda_stream
     sp = None if sd is None else sd.data_ptr()
-    if need > 0:  # a workspace one byte short is refused before any launch
+    if need > 0:  # a workspace one byte short is refused before any launch, the append's among them
+        before = cache.k.clone(), cache.v.clone()
         assert lib.wkv_prefill_gqa_shared(*args, ws.t.data_ptr(), need - 1, sp, stream) == _lib.WKV_ERR_INVALID
+        for x, y in zip(before, (cache.k, cache.v)):
+            assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
     _lib.check(lib.wkv_prefill_gqa_shared(*args, ws.t.data_ptr(), need, sp, stream), "shared prefill")
     assert_guards([ws], "shared prefill")
     return out, need

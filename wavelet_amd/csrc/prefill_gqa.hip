@@ -1131,17 +1131,17 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
   if (rc) return rc;
   WKV_CHECK_ARG(batch >= 0 && batch <= 65535, "batch must be in [0, 65535] (got %d)", batch);
   WKV_CHECK_ARG(num_tokens >= 0, "num_tokens must be >= 0");
-  if (key != nullptr || value != nullptr || slot_mapping != nullptr) {
-    // The step's new tokens go into the cache first (same stream: the
-    // attention launch below reads them back).
-    rc = cache->kv_dtype == WKV_KV_FP8_E4M3
-             ? wkv_append_fp8(cache, key, key_stride_t, key_stride_h, value, value_stride_t, value_stride_h,
-                              slot_mapping, num_tokens, stream)
-             : wkv_append(cache, key, key_stride_t, key_stride_h, value, value_stride_t, value_stride_h,
-                          slot_mapping, num_tokens, stream);
-    if (rc) return rc;
-  }
-  if (batch == 0 || max_query_len == 0) return WKV_OK;
+  // The step's new tokens go into the cache first (same stream: the attention
+  // launch below reads them back), once nothing is left to refuse.
+  auto append = [&]() -> int {
+    if (key == nullptr && value == nullptr && slot_mapping == nullptr) return WKV_OK;
+    return cache->kv_dtype == WKV_KV_FP8_E4M3
+               ? wkv_append_fp8(cache, key, key_stride_t, key_stride_h, value, value_stride_t, value_stride_h,
+                                slot_mapping, num_tokens, stream)
+               : wkv_append(cache, key, key_stride_t, key_stride_h, value, value_stride_t, value_stride_h,
+                            slot_mapping, num_tokens, stream);
+  };
+  if (batch == 0 || max_query_len == 0) return append();
   const int Hkv = cache->num_kv_heads, D = cache->head_dim, BS = cache->block_size;
   WKV_CHECK_ARG(num_q_heads > 0 && num_q_heads % Hkv == 0, "num_q_heads %d must be a multiple of num_kv_heads %d",
                 num_q_heads, Hkv);
@@ -1173,6 +1173,8 @@ static int launch_prefill(const wkv_cache_t *cache, const void *key, int64_t key
     n_wg = whole > pg.W ? whole : pg.W;
   }
   WKV_CHECK_ARG(n_wg <= INT32_MAX, "prefill grid too large");
+  rc = append();
+  if (rc) return rc;
   const dim3 grid(static_cast<unsigned>(n_wg));
   auto s = static_cast<hipStream_t>(stream);
   auto kc = static_cast<const uint8_t *>(cache->k);
