@@ -521,23 +521,28 @@ static void spread_shape(int64_t items, int max_seq, int BS, bool narrow, int *P
 // workgroups and a merge launch. 700 tokens, a layer of a captured step, two
 // workgroups -> one: d=64 bf16 2 heads, 1 / 32 / 256 sequences 8.9 / 9.7 / 23.1
 // -> 7.9 / 9.6 / 19.5 us; d=128 fp8 4 heads, the same 10.9 / 12.2 / 45.7 -> 10.2
-// / 11.3 / 39.7 us (520 to 890 tokens alike, mixed lengths more; the first with
-// 32 sequences of 890 tokens alone is slower, 11.0 -> 11.5). Wider rows keep
+// / 11.3 / 39.7 us (520 to 890 tokens alike, mixed lengths more). Wider rows keep
 // two, as one CU streams no more than about 60 bytes a ns: d=128 bf16 8 heads,
-// 8 sequences 12.0 us in two, 13.7 in one.
+// 8 sequences 12.0 us in two, 13.7 in one. So does d=64 bf16 (the most bytes of
+// the narrow rows' work per CU) past 720 tokens where 16 to 127 workgroups leave
+// the chip idle but are no longer few enough to pay for the merge launch: 8 / 32 /
+// 48 sequences of 890 tokens 10.0 / 10.5 / 11.0 in two, 10.3 / 11.3 / 11.6 in one
+// (1 and 4 sequences 9.6 / 9.8 against 8.8 / 9.6; 64 and more 12.1 against 12.0).
 // (Up to 4 partitions, eight waves in the place of four gain 6% for one sequence
 // of 500 tokens and lose 6% for 64.)
-static void choose_shape(int batch, int hkv, int max_seq, int BS, int row_bytes, int *P, int *W, int *chunks) {
+static void choose_shape(int batch, int hkv, int D, bool fp8, int max_seq, int BS, int *P, int *W, int *chunks) {
   *P = choose_partition(batch, hkv, max_seq, BS);
   decode_shape(max_seq, *P, W, chunks);
-  const bool narrow = row_bytes <= kNarrowRowBytes;
-  if (narrow && *W == 4 && *chunks == 2) {
+  const int64_t items = static_cast<int64_t>(batch) * hkv;
+  const bool narrow = (fp8 ? 2 : 4) * D <= kNarrowRowBytes;
+  if (*W == 4 && *chunks == 2) {
+    if (!narrow || (!fp8 && max_seq > 720 && items >= 16 && items < 128)) return;
     *P = ((max_seq + 7) / 8 + BS - 1) / BS * BS;
     *W = 8;
     *chunks = 1;
     return;
   }
-  spread_shape(static_cast<int64_t>(batch) * hkv, max_seq, BS, narrow, P, W, chunks);
+  spread_shape(items, max_seq, BS, narrow, P, W, chunks);
 }
 
 }  // namespace wkv
@@ -693,8 +698,7 @@ static int launch_decode(const wkv_cache_t *cache, const void *q, int64_t q_stri
   int W = 0, max_chunks = 0;
   const bool chosen = partition_size == 0;
   if (chosen) {
-    const int row_bytes = cache->kv_dtype == WKV_KV_FP8_E4M3 ? 2 * D : 4 * D;
-    choose_shape(batch, Hkv, max_seq, BS, row_bytes, &partition_size, &W, &max_chunks);
+    choose_shape(batch, Hkv, D, cache->kv_dtype == WKV_KV_FP8_E4M3, max_seq, BS, &partition_size, &W, &max_chunks);
   }
   WKV_CHECK_ARG(partition_size >= 16 && partition_size % 16 == 0, "partition_size must be a positive multiple of 16");
   WKV_CHECK_ARG((partition_size + BS - 17) / BS + 1 <= 64,
