@@ -2,12 +2,14 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 from kvcase import bits_of, check_attention, to_dev_bits
 from oracle import paged
-from wavelet_amd import PagedKVCache, paged_decode_gqa, synth
+from wavelet_amd import PagedKVCache, _lib, decode_plan, paged_decode_gqa, synth
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -61,3 +63,24 @@ def _check(cuda, hq, hkv, d, bs, lens):
     for p in (0, 128):
         got = paged.bf16_to_f32(bits_of(paged_decode_gqa(*args, partition_size=p)))
         check_attention(got, ref, f"{w.name} P={p}")
+    return w, args, ref
+
+
+@pytest.mark.parametrize("hq,hkv,d,lens", [(32, 8, 128, [4000]), (32, 8, 128, [2048, 1500]), (14, 2, 64, [2048, 33])])
+def test_a_workspace_of_the_planned_shape_is_enough(cuda, hq, hkv, d, lens):
+    """A caller that sized its workspace by decode_plan's shape (half the slots the launch would take
+    with more) is served with it, and one byte less is refused."""
+    w, (q, cache, bt, sl, scale), ref = _check(cuda, hq, hkv, d, 16, np.array(lens))
+    lib = _lib.load()
+    top = max(lens)
+    part, waves, chunks = decode_plan(w.batch, hkv, top, 16)
+    need = lib.wkv_decode_workspace_size(w.batch, hq, d, top, part * waves)
+    assert chunks > 1 and need < lib.wkv_decode_workspace_size(w.batch, hq, d, top, 0)
+    ws = torch.empty(need, dtype=torch.uint8, device=cuda)
+    out = torch.full((w.batch, hq, d), float("nan"), dtype=BF16, device=cuda)
+    args = (ctypes.byref(cache.descriptor()), q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), hq, bt.data_ptr(),
+            bt.stride(0), bt.shape[1], sl.data_ptr(), w.batch, top, ctypes.c_float(scale), 0, ws.data_ptr())
+    stream = torch.cuda.current_stream(cuda).cuda_stream
+    assert lib.wkv_paged_decode_gqa(*args, need - 1, None, stream) == _lib.WKV_ERR_INVALID
+    _lib.check(lib.wkv_paged_decode_gqa(*args, need, None, stream), "planned workspace")
+    check_attention(paged.bf16_to_f32(bits_of(out)), ref, w.name)

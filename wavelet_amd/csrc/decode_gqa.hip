@@ -718,6 +718,12 @@ static int launch_decode(const wkv_cache_t *cache, const void *q, int64_t q_stri
     WKV_CHECK_ARG(workspace != nullptr && aligned16(workspace) && workspace_bytes >= need,
                   "workspace too small: need %lld bytes, got %lld", (long long)need, (long long)workspace_bytes);
   float *part_o = static_cast<float *>(workspace);
+    // A workspace sized for wkv_decode_plan's shape and no more gets that shape.
+    if (max_chunks > 1 &&
+        workspace_bytes < wkv_decode_workspace_size(batch, num_q_heads, D, max_seq, partition_size * W)) {
+      partition_size = choose_partition(batch, Hkv, max_seq, BS);
+      decode_shape(max_seq, partition_size, &W, &max_chunks);
+    }
   float *part_ml = part_o ? part_o + static_cast<int64_t>(batch) * num_q_heads * max_chunks * D : nullptr;
   const float scale_log2 = scale * 1.4426950408889634f;
   auto s = static_cast<hipStream_t>(stream);
