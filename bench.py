@@ -466,8 +466,8 @@ def workload(args, torch, dev) -> dict:
         return {"name": name, "step": step, "w": w, "layer_bytes": attn + append, "attn_bytes": attn,
                 # the append kernel wkv_append(_fp8) picks for T = 16,384 tokens: the bulk paths
                 # from 256 (bf16) / 64 (fp8) tokens on
-                "kernel": ("prefill_gqa_kernel<128,true> (+ append_fp8_bulk_kernel)" if fp8 else
-                           "prefill_gqa_kernel<128,false> (+ append_bf16_bulk_kernel)"),
+                "kernel": ("prefill_gqa_kernel<128,true,false,false> (+ append_fp8_bulk_kernel)" if fp8 else
+                           "prefill_gqa_kernel<128,false,false,false> (+ append_bf16_bulk_kernel)"),
                 "dtype": "bf16" + (" (fp8-e4m3 KV)" if fp8 else ""),
                 "flops_per_layer": flops, "cache_bytes": caches[0].nbytes, "bound": "mfma",
                 "desc": f"Qwen3-4B prompt step: {args.layers} layers x (append + causal prefill attention), "
@@ -704,7 +704,8 @@ def main() -> int:
     if ",W,RP>" in kernel_name:  # the GQA decode: the library's waves per workgroup for this geometry
         from wavelet_amd import decode_plan
 
-        _, waves, _ = decode_plan(w.batch, w.num_kv_heads, int(w.context_lens.max()), w.block_size, args.partition)
+        _, waves, _ = decode_plan(w.batch, w.num_kv_heads, int(w.context_lens.max()), w.block_size, args.partition,
+                                  head_dim=w.head_dim, kv_dtype=wl["kv_dtype"])
         # read policy: 0 cached (shared blocks), 1 streamed, 2 the group split (prompt cached, own tokens streamed)
         rp = 2 if getattr(step, "grouped", False) else (1 if wl["stream"] else 0)
         kernel_name = kernel_name.replace(",W,RP>", f",{waves},{rp}>")

@@ -219,18 +219,28 @@ int wkv_grouped_decode_order(const int32_t *seq_lens, int32_t batch, int32_t gro
                              int32_t max_seq_len, int32_t block_size, int32_t partition_size, int32_t *order,
                              void *stream);
 
-/* The launch shape the two GQA decode calls use for this geometry (host
- * only, no GPU): the partition size (partition_size, or the library's choice
- * when 0), the waves per workgroup and the workgroups (chunks) per sequence
- * and KV head; more than one chunk leaves partials for the merge kernel. (The
- * library's choice is adapted to the cache and the chip at the launch: two
- * chunks of four waves go as one of eight for fp8 or d=64 caches, several
- * chunks of eight waves that would leave CUs idle as more chunks of four;
- * one chunk never becomes several, and the workspace need stays within
- * wkv_decode_workspace_size of partition 0.) For planning and labelling; no reference counterpart. max_seq_len is the one
- * the decode call will get, clipped to the block-table width. */
+/* The shape of the two GQA decode calls by lengths alone (host only, no GPU):
+ * the partition size (partition_size, or the library's choice when 0), the
+ * waves per workgroup and the workgroups (chunks) per sequence and KV head;
+ * more than one chunk leaves partials for the merge kernel. A given partition
+ * is launched so; the library's choice is adapted to the cache and the chip at
+ * the launch (wkv_decode_launch_plan). A workspace for this shape is always
+ * enough: without room for the adapted one, this one is launched. No reference
+ * counterpart. max_seq_len is the one the decode call will get, clipped to the
+ * block-table width. */
 int wkv_decode_plan(int32_t batch, int32_t num_kv_heads, int32_t max_seq_len, int32_t block_size,
                     int32_t partition_size, int32_t *out_partition, int32_t *out_waves, int32_t *out_chunks);
+
+/* The shape the two GQA decode calls launch for a cache of this head size and
+ * type (host only, no GPU), with the workspace of wkv_decode_workspace_size for
+ * the same partition_size: wkv_decode_plan's, except where the library chooses
+ * (partition_size 0) and two chunks of four waves go as one of eight (fp8 or
+ * d=64 caches), or several chunks of eight waves that would leave CUs idle as
+ * more chunks of four. One chunk never becomes several. For planning and
+ * labelling; no reference counterpart. */
+int wkv_decode_launch_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, int32_t kv_dtype,
+                           int32_t max_seq_len, int32_t block_size, int32_t partition_size, int32_t *out_partition,
+                           int32_t *out_waves, int32_t *out_chunks);
 
 /* One whole decode step of one layer in one launch: append token b of
  * key/value ([batch, num_kv_heads, head_dim] bf16) at slot_mapping[b] (-1 =

@@ -187,6 +187,49 @@ def test_decode_plan_shapes_and_errors():
     assert lib.wkv_decode_plan(64, 8, 4096, 16, 0, None, ctypes.byref(o), ctypes.byref(o)) == _lib.WKV_ERR_INVALID
 
 
+def test_decode_launch_plan_is_what_each_cache_gets():
+    """The library's choice for a head size and type, on both sides of each bound of the launch rules; a
+    given partition, one chunk and full chips keep the plain shape."""
+    from wavelet_amd import decode_plan
+
+    def launch(b, hkv, n, bs, d, kv, part=0):
+        return decode_plan(b, hkv, n, bs, part, head_dim=d, kv_dtype=kv)
+
+    # 5 to 7 partitions of narrow rows: one workgroup of eight waves
+    for n in (512, 513, 700, 720, 721, 896, 897):
+        plain = decode_plan(1, 2, n, 16)
+        one = ((n + 7) // 8 + 15) // 16 * 16, 8, 1
+        inside = 512 < n <= 896
+        assert plain == ((128, 4, 2) if inside else (128, 4, 1) if n == 512 else (128, 8, 1))
+        assert launch(1, 2, n, 16, 128, "bf16") == plain
+        for d, kv in ((64, "bf16"), (64, "fp8_e4m3"), (128, "fp8_e4m3")):
+            assert launch(1, 2, n, 16, d, kv) == (one if inside else plain)
+            assert launch(1, 2, n, 16, d, kv, 128) == plain
+    # ... but d=64 bf16 past 720 tokens with 16 to 127 (sequence, head) pairs
+    for pairs, two in ((15, False), (16, True), (127, True), (128, False)):
+        assert (launch(pairs, 1, 800, 16, 64, "bf16")[2] == 2) == two
+        assert launch(pairs, 1, 720, 16, 64, "bf16")[2] == launch(pairs, 1, 800, 16, 64, "fp8_e4m3")[2] == 1
+    # few long contexts: more workgroups of four waves
+    assert launch(1, 8, 1024, 16, 128, "bf16") == (128, 8, 1)
+    assert launch(1, 8, 1025, 16, 128, "bf16") == (64, 4, 5)
+    assert launch(1, 8, 4096, 16, 128, "bf16") == launch(1, 8, 4096, 16, 128, "fp8_e4m3") == (128, 4, 8)
+    assert launch(1, 8, 4097, 16, 128, "bf16") == (128, 4, 9)  # nine slots: wide rows only
+    assert launch(1, 8, 4097, 16, 128, "fp8_e4m3") == decode_plan(1, 8, 4097, 16) == (128, 8, 5)
+    assert launch(4, 8, 2048, 16, 128, "bf16") == (64, 4, 8)  # 4 x 8 x 8 workgroups: one per CU
+    assert launch(5, 8, 2048, 16, 128, "bf16") == (128, 4, 4)  # partitions of 64 would be more
+    assert launch(9, 8, 2048, 16, 128, "bf16") == decode_plan(9, 8, 2048, 16) == (128, 8, 2)
+    for args in ((64, 8, 4096, 16), (64, 8, 65536, 16)):
+        assert launch(*args, 128, "bf16") == decode_plan(*args)
+    with pytest.raises(ValueError):
+        decode_plan(1, 8, 4096, 16, head_dim=128)
+    lib = _lib.load()
+    o = ctypes.byref(ctypes.c_int32())
+    assert lib.wkv_decode_launch_plan(1, 8, 96, 0, 4096, 16, 0, o, o, o) == _lib.WKV_ERR_INVALID
+    assert lib.wkv_decode_launch_plan(1, 8, 128, 2, 4096, 16, 0, o, o, o) == _lib.WKV_ERR_INVALID
+    assert lib.wkv_decode_launch_plan(1, 8, 128, 0, 4096, 8, 0, o, o, o) == _lib.WKV_ERR_INVALID
+    assert lib.wkv_decode_launch_plan(1, 8, 128, 0, 4096, 16, 0, o, None, o) == _lib.WKV_ERR_INVALID
+
+
 @host_only
 def test_prefill_rejects_bad_arguments_before_launch():
     lib = _lib.load()

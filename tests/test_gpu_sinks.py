@@ -78,7 +78,7 @@ def test_decode_sinks_match_oracle(cuda, hq, hkv, d):
         plain = paged.decode_gqa(qf, kf, vf, w.block_tables, w.context_lens, w.scale)
         assert np.abs(ref - plain).max() > 0.1, "the sinks must matter in this case"
         for p in parts:
-            shapes.add(decode_plan(w.batch, hkv, int(lens.max()), w.block_size, p)[1:])
+            shapes.add(decode_plan(w.batch, hkv, int(lens.max()), w.block_size, p, head_dim=d, kv_dtype="bf16")[1:])
             out = paged_decode_gqa(qd, cache, bt, sl, w.scale, partition_size=p, sinks=sd)
             got = paged.bf16_to_f32(bits_of(out))
             a, r = check_attention(got, ref, f"{w.name} sinks P={p}")

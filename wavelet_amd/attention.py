@@ -63,16 +63,24 @@ def _max_len(seq_lens: torch.Tensor, max_seq_len: int | None) -> int:
     return int(seq_lens.max().item()) if seq_lens.numel() else 0
 
 
-def decode_plan(batch: int, num_kv_heads: int, max_seq_len: int, block_size: int,
-                partition_size: int = 0) -> tuple[int, int, int]:
-    """(partition size, waves per workgroup, workgroups per sequence and KV head)
-    that ``paged_decode_gqa`` launches for this geometry (host-side, no GPU). The launch adapts
-    a chosen shape to the cache and the chip (include/wkv.h): (.., 4, 2) to one workgroup of eight waves for
-    narrow rows, several workgroups of eight waves to more of four for few sequences."""
+def decode_plan(batch: int, num_kv_heads: int, max_seq_len: int, block_size: int, partition_size: int = 0, *,
+                head_dim: int | None = None, kv_dtype: str | None = None) -> tuple[int, int, int]:
+    """(partition size, waves per workgroup, workgroups per sequence and KV head) of a decode step
+    (host-side, no GPU). With ``head_dim`` and ``kv_dtype`` of the caches: what ``paged_decode_gqa``
+    launches for them. Without: the shape by lengths alone, which a launch whose partition is the library's
+    choice adapts to the cache and the chip (include/wkv.h)."""
+    if (head_dim is None) != (kv_dtype is None):
+        raise ValueError("head_dim and kv_dtype go together")
     p, w, c = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
-    _lib.check(_lib.load().wkv_decode_plan(int(batch), int(num_kv_heads), int(max_seq_len), int(block_size),
-                                           int(partition_size), ctypes.byref(p), ctypes.byref(w), ctypes.byref(c)),
-               "decode_plan")
+    out = (ctypes.byref(p), ctypes.byref(w), ctypes.byref(c))
+    lib = _lib.load()
+    if head_dim is None:
+        rc = lib.wkv_decode_plan(int(batch), int(num_kv_heads), int(max_seq_len), int(block_size), int(partition_size),
+                                 *out)
+    else:
+        rc = lib.wkv_decode_launch_plan(int(batch), int(num_kv_heads), int(head_dim), KV_DTYPES[kv_dtype],
+                                        int(max_seq_len), int(block_size), int(partition_size), *out)
+    _lib.check(rc, "decode_plan")
     return p.value, w.value, c.value
 
 

@@ -565,6 +565,22 @@ extern "C" int wkv_decode_plan(int32_t batch, int32_t num_kv_heads, int32_t max_
   return WKV_OK;
 }
 
+extern "C" int wkv_decode_launch_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, int32_t kv_dtype,
+                                      int32_t max_seq_len, int32_t block_size, int32_t partition_size,
+                                      int32_t *out_partition, int32_t *out_waves, int32_t *out_chunks) {
+  WKV_CHECK_ARG((head_dim == 64 || head_dim == 128) && (kv_dtype == WKV_KV_BF16 || kv_dtype == WKV_KV_FP8_E4M3),
+                "head_dim must be 64 or 128 and kv_dtype bf16 or fp8_e4m3");
+  const int rc = wkv_decode_plan(batch, num_kv_heads, max_seq_len, block_size, partition_size, out_partition, out_waves,
+                                 out_chunks);
+  if (rc || partition_size != 0) return rc;
+  int P, W, chunks;
+  choose_shape(batch, num_kv_heads, head_dim, kv_dtype == WKV_KV_FP8_E4M3, max_seq_len, block_size, &P, &W, &chunks);
+  *out_partition = P;
+  *out_waves = W;
+  *out_chunks = chunks;
+  return WKV_OK;
+}
+
 extern "C" int64_t wkv_decode_workspace_size(int32_t batch, int32_t num_q_heads, int32_t head_dim,
                                              int32_t max_seq_len, int32_t partition_size) {
   if (batch < 0 || num_q_heads <= 0 || head_dim <= 0 || max_seq_len < 0 || partition_size < 0) return -1;

@@ -260,15 +260,15 @@ class GraphDecodeStep:
         batch = step.seq_lens.shape[0]
         # the launch's partition, waves per workgroup and chunks: partials (and the scratch)
         # only when a context spans more than one workgroup
-        c0 = caches[0]
         bt_width = step.block_table.shape[1]
-        part, waves, chunks = decode_plan(batch, c0.num_kv_heads, min(step.max_seq_len, bt_width * c0.block_size),
-                                          c0.block_size, step.partition_size)
-        need = lib.wkv_decode_workspace_size(batch, q[0].shape[1], c0.head_dim,
-                                             min(step.max_seq_len, bt_width * c0.block_size), part * waves)
-        if chunks > 1 and (need < 0 or need > _lib.WKV_NOALLOC_SCRATCH_BYTES):
-            raise ValueError(f"the step's split-K partials need {need} bytes, beyond the "
-                             f"{_lib.WKV_NOALLOC_SCRATCH_BYTES}-byte scratch of the allocation-free decode")
+        for qq, c in zip(q, caches):
+            msl = min(step.max_seq_len, bt_width * c.block_size)
+            part, waves, chunks = decode_plan(batch, c.num_kv_heads, msl, c.block_size, step.partition_size,
+                                              head_dim=c.head_dim, kv_dtype=c.kv_dtype)
+            need = lib.wkv_decode_workspace_size(batch, qq.shape[1], c.head_dim, msl, part * waves)
+            if chunks > 1 and (need < 0 or need > _lib.WKV_NOALLOC_SCRATCH_BYTES):
+                raise ValueError(f"the step's split-K partials need {need} bytes, beyond the "
+                                 f"{_lib.WKV_NOALLOC_SCRATCH_BYTES}-byte scratch of the allocation-free decode")
         dev = caches[0].device
         self._live = step._live
         self._live.check_all()
