@@ -251,6 +251,34 @@ def _expected_grouped_order(lens, gs, hkv, max_seq, bs, partition):
     return out, n
 
 
+@pytest.mark.parametrize("batch,gs,hkv,max_seq,bs,n_cls", [
+    (48, 3, 1, 700, 16, 8),   # two workgroups per sequence, or one for narrow rows
+    (16, 4, 2, 700, 16, 4),
+    (24, 3, 1, 2000, 16, 4),  # spread to eight workgroups of partitions of 64; two in the plain shape
+    (8, 2, 2, 5000, 16, 4),   # wide rows spread to ten workgroups, narrow rows keep five
+    (16, 2, 1, 7000, 16, 8),  # wide rows 14, narrow rows seven
+    (9, 3, 1, 7000, 16, 1),   # eight classes would be unequal
+])
+def test_grouped_decode_order_suits_every_cache(cuda, batch, gs, hkv, max_seq, bs, n_cls):
+    """The order is made without the cache: whatever shape its head size and type are launched in, a group's
+    members lie at positions of one residue modulo that shape's classes; longest first within a class."""
+    rng = np.random.default_rng(batch)
+    lens = rng.integers(1, max_seq + 1, batch).astype(np.int32)
+    got = grouped_decode_order(torch.from_numpy(lens).to(cuda), gs, hkv, max_seq, bs, 0).cpu().numpy()
+    assert sorted(got) == list(range(batch))
+    where = np.argsort(got)
+    for d, kv in ((64, "bf16"), (128, "bf16"), (64, "fp8_e4m3"), (128, "fp8_e4m3")):
+        chunks = decode_plan(batch, hkv, max_seq, bs, head_dim=d, kv_dtype=kv)[2]
+        n = 8 // math.gcd(8, chunks * hkv)
+        assert n <= n_cls or n_cls == 1
+        if n_cls > 1:
+            assert all(len({where[i] % n for i in range(g, g + gs)}) == 1 for g in range(0, batch, gs)), (d, kv)
+    for c in range(n_cls):
+        ranked = lens[got[c::n_cls]]
+        assert (np.diff(ranked) <= 0).all()
+        assert n_cls == 1 or {(i // gs) % n_cls for i in got[c::n_cls]} == {c}
+
+
 @pytest.mark.parametrize("batch,gs,hkv,max_seq,part,n_cls", [
     (256, 8, 4, 4096, 0, 2),   # Qwen2.5-7B groups: one workgroup per (sequence, KV head)
     (48, 3, 1, 1000, 0, 8),    # one KV head: eight classes

@@ -667,20 +667,23 @@ static int order_classes(int workgroups, int batch, int group_size) {
   return batch % (group_size * n_cls) == 0 ? n_cls : 1;
 }
 
+// The order is made without the cache, whose type and head size the launch's
+// shape depends on (choose_shape): the most classes of any shape it may have. All
+// are powers of two, so positions that agree modulo the most agree modulo the
+// others' as well, and groups stay together whichever shape is launched.
 static int grouped_order_classes(int batch, int group_size, int hkv, int max_seq, int BS, int partition_size) {
   int P = partition_size != 0 ? partition_size : choose_partition(batch, hkv, max_seq, BS);
   int W, chunks;
   decode_shape(max_seq, P, &W, &chunks);
-  if (partition_size == 0 && W == 8) {
-    spread_shape(static_cast<int64_t>(batch) * hkv, max_seq, BS, true, &P, &W, &chunks);
-  } else if (partition_size == 0 && W == 4 && chunks == 2) {
-    // Two workgroups per sequence and head, or one for narrow rows (choose_shape; the order is
-    // made without the cache): a position's residue modulo the classes of one gives its residue
-    // modulo those of two, so the order of one keeps groups together in both.
-    const int n = order_classes(hkv, batch, group_size);
-    if (n > 1) return n;
+  int n = order_classes(chunks * hkv, batch, group_size);
+  if (partition_size == 0) {
+    for (int cache = 0; cache < 4; ++cache) {
+      choose_shape(batch, hkv, cache & 1 ? 128 : 64, (cache & 2) != 0, max_seq, BS, &P, &W, &chunks);
+      const int c = order_classes(chunks * hkv, batch, group_size);
+      n = c > n ? c : n;
+    }
   }
-  return order_classes(chunks * hkv, batch, group_size);
+  return n;
 }
 
 static int launch_decode(const wkv_cache_t *cache, const void *q, int64_t q_stride_b, int64_t q_stride_h, void *out,
@@ -715,6 +718,12 @@ static int launch_decode(const wkv_cache_t *cache, const void *q, int64_t q_stri
   const bool chosen = partition_size == 0;
   if (chosen) {
     choose_shape(batch, Hkv, D, cache->kv_dtype == WKV_KV_FP8_E4M3, max_seq, BS, &partition_size, &W, &max_chunks);
+    // A workspace sized for wkv_decode_plan's shape and no more gets that shape.
+    if (max_chunks > 1 &&
+        workspace_bytes < wkv_decode_workspace_size(batch, num_q_heads, D, max_seq, partition_size * W)) {
+      partition_size = choose_partition(batch, Hkv, max_seq, BS);
+      decode_shape(max_seq, partition_size, &W, &max_chunks);
+    }
   }
   WKV_CHECK_ARG(partition_size >= 16 && partition_size % 16 == 0, "partition_size must be a positive multiple of 16");
   WKV_CHECK_ARG((partition_size + BS - 17) / BS + 1 <= 64,
@@ -734,12 +743,6 @@ static int launch_decode(const wkv_cache_t *cache, const void *q, int64_t q_stri
     WKV_CHECK_ARG(workspace != nullptr && aligned16(workspace) && workspace_bytes >= need,
                   "workspace too small: need %lld bytes, got %lld", (long long)need, (long long)workspace_bytes);
   float *part_o = static_cast<float *>(workspace);
-    // A workspace sized for wkv_decode_plan's shape and no more gets that shape.
-    if (max_chunks > 1 &&
-        workspace_bytes < wkv_decode_workspace_size(batch, num_q_heads, D, max_seq, partition_size * W)) {
-      partition_size = choose_partition(batch, Hkv, max_seq, BS);
-      decode_shape(max_seq, partition_size, &W, &max_chunks);
-    }
   float *part_ml = part_o ? part_o + static_cast<int64_t>(batch) * num_q_heads * max_chunks * D : nullptr;
   const float scale_log2 = scale * 1.4426950408889634f;
   auto s = static_cast<hipStream_t>(stream);
