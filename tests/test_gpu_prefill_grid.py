@@ -9,7 +9,7 @@ from kvcase import bits_of, check_attention, to_dev_bits
 from oracle import fp8, paged
 from test_gpu_prefill import BF16, _case, _run_and_check
 from test_gpu_prefill_shared import _reference, _shared_call
-from wavelet_amd import _lib, prefill_gqa
+from wavelet_amd import PagedKVCache, _lib, prefill_gqa
 from wavelet_amd.cache import KV_DTYPES
 from wavelet_amd.plan import PrefillStep
 
@@ -120,6 +120,29 @@ def test_layers_of_a_plan_take_turns_with_its_workspace(cuda, kv_dtype):
         step.run()
     for i, (wl, cache, host, new) in enumerate(layers):
         check_attention(paged.bf16_to_f32(bits_of(outs[i])), _reference(wl, cache, host, new), f"layer {i}")
+
+
+def test_layers_of_different_block_sizes_share_a_plan(cuda):
+    """One table over caches of 16- and 64-token blocks: the second layer's launch sees four times the keys, and
+    the plan's workspace is sized for it."""
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(1)
+    rnd = lambda *shape: torch.randn(shape, generator=gen, device=cuda).to(BF16)  # noqa: E731
+    caches = [PagedKVCache(100, bs, 8, 128, device=cuda) for bs in (16, 64)]
+    for c in caches:
+        c.k.copy_(rnd(*c.k.shape))
+        c.v.copy_(rnd(*c.v.shape))
+    q, k, v = ([rnd(1, h, 128) for _ in caches] for h in (32, 8, 8))
+    outs = [torch.empty_like(x) for x in q]
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=cuda)  # noqa: E731
+    bt = torch.arange(100, dtype=torch.int32, device=cuda).view(1, 100)
+    slots = torch.tensor([1499], device=cuda)
+    needs = [_lib.load().wkv_prefill_workspace_size(1, 0, 8, 32, 128, 1, min(6000, 100 * c.block_size), 0) for c in caches]
+    assert 0 < needs[0] < needs[1]
+    step = PrefillStep(caches, q, k, v, outs, bt, i32(1500), i32(0, 1), slots, 0.1, 1, 6000)
+    step.run()
+    for c, qq, oo in zip(caches, q, outs):
+        assert torch.equal(oo, prefill_gqa(qq, c, bt, i32(1500), i32(0, 1), 0.1, max_query_len=1, max_seq_len=6000))
 
 
 @pytest.mark.parametrize("kv_dtype", ["bf16", "fp8_e4m3"])

@@ -411,10 +411,9 @@ class PrefillStep:
         T = slot_mapping.numel()
         self.lib = lib = _lib.load()
         self.stream = torch.cuda.current_stream(dev).cuda_stream
-        c0 = caches[0]
         need = max(lib.wkv_prefill_workspace_size(
             batch, KV_DTYPES[c.kv_dtype], c.num_kv_heads, qq.shape[1], c.head_dim, int(max_query_len),
-            min(int(max_seq_len), self.block_table.shape[1] * c0.block_size), 0) for c, qq in zip(caches, q))
+            min(int(max_seq_len), self.block_table.shape[1] * c.block_size), 0) for c, qq in zip(caches, q))
         # the plan's own scratch for a small grid's shared key ranges (None: nothing is shared)
         self.workspace = torch.empty(need, dtype=torch.uint8, device=dev) if need > 0 else None
         split = (0, self.workspace.data_ptr(), need, None) if need > 0 else (0, None, 0, None)
