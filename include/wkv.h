@@ -377,9 +377,16 @@ int wkv_prefill_gqa_sinks(const wkv_cache_t *cache, const void *key, int64_t key
  * evenly over the chip's workgroups: a query tile whose keys fall to several
  * workgroups leaves fp32 partials in the workspace and a second kernel merges
  * them by log-sum-exp. Otherwise the arguments, result and behaviour of
- * wkv_prefill_gqa (of wkv_prefill_gqa_sinks with sinks non-NULL).
+ * wkv_prefill_gqa (of wkv_prefill_gqa_sinks with sinks non-NULL), but for a
+ * row's last bits: where its keys are cut follows the lengths of every sequence
+ * of the call, and each part takes its bf16 probabilities against its own
+ * maximum (the error against float64 is the same, 0.0024 relative). Without a
+ * workspace a row's bits depend on its own sequence alone.
  * workgroups: 0 = the library's choice (sharing only where it is expected to
- * be faster), n > 0 = share over n (rounded up to a multiple of 8; ignored for
+ * be faster: the host decides by max_query_len and max_seq_len whether a launch
+ * may share, and the launch by the lengths themselves whether it does. A bound
+ * of thousands of keys over contexts of hundreds costs about 4 us, the length
+ * sums and an empty merge launch), n > 0 = share over n (rounded up to a multiple of 8; ignored for
  * launches of more than 1,024 groups of four 32-query tiles per KV head).
  * workspace: wkv_prefill_workspace_size() bytes for the same geometry and
  * workgroups, max_seq_len clipped to the block-table width (0 bytes = nothing

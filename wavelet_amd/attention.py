@@ -335,7 +335,9 @@ def prefill_gqa(
     the new tokens are appended first (``cache.append``) and attended from the
     cache -- the prompt step of ``llm.generate`` (wavelet/inference/
     engine.py:887). ``max_query_len`` / ``max_seq_len`` (host ints) avoid
-    device syncs when given. ``sinks`` as for ``paged_decode_gqa``.
+    device syncs when given; they are upper bounds, and the launch is chosen by them (loose ones cost
+    a few microseconds: include/wkv.h, ``wkv_prefill_gqa_shared``). A row's last bits may depend on the
+    other sequences of the call, as for ``paged_decode_gqa``. ``sinks`` as for ``paged_decode_gqa``.
     """
     if not isinstance(cache, PagedKVCache):
         raise ValueError("cache must be a PagedKVCache")

@@ -366,7 +366,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(FP8 ? 4 
 // `slots` (Slots gives the counts; false = the decode kernel finished the row).
 // The loads of the first slots go out before the counts are known (their
 // addresses do not depend on them; unused slots are masked, never summed), so
-// a row costs about one memory round trip.
+// a row of up to SPEC slots costs about one memory round trip; each slot past
+// them two more (its weight, then its output).
 template <int D, typename Slots>
 __global__ __launch_bounds__(256) void merge_partials_kernel(const float *__restrict__ part_o,
                                                              const float *__restrict__ part_ml,

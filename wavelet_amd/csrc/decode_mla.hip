@@ -794,12 +794,12 @@ static int launch_mla(const wkv_mla_cache_t *cache, const void *q_nope, int64_t 
   auto qn = static_cast<const uint16_t *>(q_nope);
   auto qpp = static_cast<const uint16_t *>(q_pe);
   auto oo = static_cast<uint16_t *>(out);
-#define WKV_MLA(NQv)                                                                                        \
-  decode_mla_kernel<NQv><<<grid, mla_threads<NQv>(), 0, s>>>(lat, qn, qn_stride_b, qn_stride_h, qpp, qp_stride_b,          \
-                                                    qp_stride_h, oo, part_o, part_ml, block_table, bt_stride,      \
-                                                    max_blocks_per_seq, max_seq, seq_lens, BS, cache->num_blocks, \
-                                                    scale_log2, partition_size, max_parts, num_heads, batch, ap,  \
-                                                    batch % 8 == 0, sinks)
+#define WKV_MLA(NQv)                                                                                              \
+  decode_mla_kernel<NQv><<<grid, mla_threads<NQv>(), 0, s>>>(lat, qn, qn_stride_b, qn_stride_h, qpp, qp_stride_b, \
+                                                             qp_stride_h, oo, part_o, part_ml, block_table,       \
+                                                             bt_stride, max_blocks_per_seq, max_seq, seq_lens,    \
+                                                             BS, cache->num_blocks, scale_log2, partition_size,   \
+                                                             max_parts, num_heads, batch, ap, batch % 8 == 0, sinks)
   switch (num_heads) {
     case 16: WKV_MLA(1); break;
     case 32: WKV_MLA(2); break;

@@ -589,8 +589,8 @@ extern "C" int wkv_mla_append(const wkv_mla_cache_t *cache, const void *kv_c, in
 }
 
 static int launch_gather(const wkv_cache_t *cache, const int32_t *block_table, int64_t bt_stride,
-                          int32_t max_blocks_per_seq, const int32_t *seq_lens, const int64_t *cu_seq_lens,
-                          int32_t batch, void *out_k, void *out_v, int32_t dequant, void *stream) {
+                         int32_t max_blocks_per_seq, const int32_t *seq_lens, const int64_t *cu_seq_lens, int32_t batch,
+                         void *out_k, void *out_v, int32_t dequant, void *stream) {
   int rc = check_cache(cache, -1);
   if (rc) return rc;
   WKV_CHECK_ARG(batch >= 0 && batch <= 65535, "batch must be in [0, 65535]");

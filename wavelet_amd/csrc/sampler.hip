@@ -295,10 +295,9 @@ constexpr int kMaxHits = 2048;
 // together, or one of them, for which the radix select runs once (8,000 tokens,
 // 128 rows, top_k 200: 22.0 us ranked, 18.8 by radix; top_k 20: 16.6 and 18.0).
 constexpr int kRanked = 256, kRankedOne = 128;
-// Draws a wave may hold back before making them 64 at a time (general final pass).
-constexpr int kQueue = 128;
-// The same for the final pass's fast loop, which makes its draws after every
-// fourth token slot: fewer than 64 pending, plus 64 per slot.
+// Draws a wave may hold back before making them 64 at a time: the final pass's
+// fast loop makes them after every fourth token slot, so fewer than 64 pending
+// and 64 per slot (its general loop holds fewer than 128).
 constexpr int kFastQueue = 64 + 4 * 64;
 static_assert(kBins == 2 * kSampleThreads, "the threshold scan gives every thread two bins");
 

@@ -387,7 +387,8 @@ class PrefillStep:
 
     ``q[l]`` ``[T, Hq, D]``, ``key[l]`` / ``value[l]`` ``[T, Hkv, D]`` and
     ``out[l]`` are layer ``l``'s buffers; ``cu_seqlens_q [B+1]`` int32 splits
-    the ``T`` rows by sequence and ``slot_mapping [T]`` places them.
+    the ``T`` rows by sequence and ``slot_mapping [T]`` places them. ``max_query_len`` and
+    ``max_seq_len`` are upper bounds of the lengths in the buffers, as for ``prefill_gqa``.
     """
 
     def __init__(self, caches: list[PagedKVCache], q: list[torch.Tensor], key: list[torch.Tensor],

@@ -76,7 +76,9 @@ def sample(
     int32 bitmap of the kept set (``mask_token_ids`` lists it) and ``counts``
     its sizes, both ``None`` unless ``return_mask``. ``out`` may hold those four
     outputs, preallocated (mask and counts may be ``None`` without
-    ``return_mask``): a serving loop then allocates nothing per step.
+    ``return_mask``): a serving loop that also gives its parameters as tensors then allocates nothing per step,
+    but for the scratch of rows cut into slices (768 bytes a row, from the caching allocator: up to 128 rows drawn
+    from the whole of a vocabulary above 40,960, ``top_k``, ``top_p`` and ``min_p`` all ``None``).
     """
     for name, v in (("temperature", temperature), ("top_p", top_p), ("min_p", min_p),
                     ("repetition_penalty", repetition_penalty)):
