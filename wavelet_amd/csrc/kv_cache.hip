@@ -270,7 +270,9 @@ __device__ __forceinline__ int64_t lens_before(const int32_t *__restrict__ lens,
 // Gather: one workgroup per (sequence, block index), reading whole blocks and
 // writing whole rows of the contiguous [tokens, H, D] output. Bound by HBM: 18,000 tokens of 8 heads (147 MB) take
 // 28 us, inputs in the caches, 34 from HBM (41 with V read an element at a time
-// and K written 16 bytes to a row). cu = nullptr: sequence i starts at the
+// and K written 16 bytes to a row). Blocks of few heads leave most of a round
+// without pieces, and issue no loads for them (2,000 sequences of 1 to 64 tokens,
+// 2 heads of 64: bf16 19.1 -> 17.2 us, fp8 16.8 -> 13.9). cu = nullptr: sequence i starts at the
 // sum of the lengths before it, which each wave adds up itself (a few loads
 // beside the block id's) -- the prefix sum as launches of its own cost the
 // call 7.7 us more.
@@ -302,7 +304,8 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint8_t *__restrict__
     u32x4 raw[KB];
 #pragma unroll
     for (int k = 0; k < KB; ++k) {
-      const int w = w0 + 256 * k < nk ? w0 + 256 * k : w0;
+      const int w = w0 + 256 * k;
+      if (w >= nk) break;
       const int c = w % C, ho = w / C, h = ho / ntok, o = ho - h * ntok;
       raw[k] = *reinterpret_cast<const u32x4 *>(kc + ((((blk * H + h) * C + c) * BS + o) * 16));
     }
@@ -347,6 +350,7 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint8_t *__restrict__
     u32x4 raw[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
+      if (q0 + 256 * k / (D * PR) >= H * ng) break;  // uniform: no tile left (256 threads take whole tiles)
       const int i = threadIdx.x + 256 * k;
       const int q = q0 + i / (D * PR) < H * ng ? q0 + i / (D * PR) : q0;
       const int h = q / ng, g = q - h * ng, d = i / PR % D;
@@ -354,6 +358,7 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint8_t *__restrict__
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
+      if (q0 + 256 * k / (D * PR) >= H * ng) break;
       const int i = threadIdx.x + 256 * k;
       uint32_t *l = reinterpret_cast<uint32_t *>(&lv[(i / PR) * RP + 16 * (i % PR)]);
 #pragma unroll
@@ -362,6 +367,7 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint8_t *__restrict__
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < VT * PT / 256; ++k) {
+      if (q0 + 256 * k / PT >= H * ng) break;
       const int i = threadIdx.x + 256 * k;
       const int t = i / PT, o = i % PT / (D / E), d0 = i % (D / E) * E;
       const int q = q0 + t;
