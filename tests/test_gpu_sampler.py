@@ -106,13 +106,29 @@ def test_sampler_capture_paths(cuda):
 
 
 def test_sampler_vocab_beyond_lds_mask(cuda):
-    """300,000 tokens (9,375 mask words): the list path keeps the full-row final pass."""
+    """300,000 tokens (9,375 mask words): the list path builds its mask in two turns."""
     V = 300000
     rows = [(0.7, 50, 0.9, 0.0, 1.0), (1.0, 0, 0.9, 0.0, 1.0), (1.0, 0, 1.0, 0.0, 1.0)]
     x = (synth.normal(synth.stream_key("smp-300k"), len(rows) * V) * 40.0).astype(np.float32).reshape(len(rows), V)
     seen_lists = [np.zeros(0, np.int64) for _ in rows]
     seeds = np.arange(len(rows), dtype=np.int64) + 5
     _check_rows(cuda, x, rows, seen_lists, seeds, 1, torch.bfloat16)
+
+
+@pytest.mark.parametrize("vocab", [262144, 262145, 524297])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_group_sizes_and_masks_of_long_rows(cuda, vocab, dtype):
+    """Groups of 4, 8 and 16 chunks a thread and masks of one to three turns: top_k, top_p and min_p whose lists
+    fill, overflow and (min_p) spread over more groups than are read again; the last token kept."""
+    rows = [(1.0, 50, 1.0, 0.0, 1.0), (0.7, 50, 0.9, 0.0, 1.1), (1.0, 1000, 0.95, 0.0, 1.0), (1.0, 1, 1.0, 0.0, 1.0),
+            (0.0, 20, 1.0, 0.0, 1.0), (1.0, 0, 0.9, 0.0, 1.0), (1.0, 0, 1.0, 0.3, 1.0), (1.0, 0, 1.0, 1e-6, 1.0)]
+    x = (synth.normal(synth.stream_key("smp-long", vocab), len(rows) * vocab) * 3.0).astype(np.float32)
+    x = x.reshape(len(rows), vocab)
+    x[:, vocab - 1] = 16.0
+    x[2] = np.round(x[2])  # thousands of ties at the threshold
+    rng = np.random.default_rng(vocab)
+    _check_rows(cuda, x, rows, [rng.integers(0, vocab, 300) for _ in rows], np.arange(len(rows), dtype=np.int64) + 3, 2,
+                dtype)
 
 
 def test_sampler_draws_match_kept_softmax(cuda):

@@ -283,14 +283,16 @@ constexpr int kCand = 4096;
 // A token this many bins or more below the maximum (22.2 nats) weighs under
 // one unit of fixed_mass: exactly 0.
 constexpr int kMassBins = 711;
-// Rows of up to kMaskWords * 32 tokens build their mask in LDS on the list
-// path, and keep their group maxima.
+// Mask words that the list path builds in LDS at a time (longer rows take turns).
 constexpr int kMaskWords = 8192;
-constexpr int kGroup = 4;  // chunks per group
-constexpr int kGroups = kMaskWords * 32 / (kGroup * kStep8);
-// More groups to read again than this (of up to kGroups x 1,024): a pass over
-// the row is as cheap.
-constexpr int kMaxHits = 2048;
+// A thread's groups: 2^kGroupShift chunks each up to 262,144 tokens, doubled
+// for longer rows until kGroups of them cover the row (300,000 bf16 tokens, 1 /
+// 256 rows, against whole passes: top_k 50 with top_p 81.9 / 101.4 -> 26.7 /
+// 39.6 us, min_p 46.0 / 61.7 -> 21.0 / 34.5).
+constexpr int kGroups = 8, kGroupShift = 2;
+// More chunks to read again than this under min_p (of up to kGroups x 1,024
+// groups): a pass over the row is as cheap.
+constexpr int kMaxHitChunks = 8192;
 // Entries of a list whose thresholds are found by ranking: top_k and top_p
 // together, or one of them, for which the radix select runs once (8,000 tokens,
 // 128 rows, top_k 200: 22.0 us ranked, 18.8 by radix; top_k 20: 16.6 and 18.0).
@@ -322,6 +324,7 @@ struct SampleArgs {
   float *logprobs;           // [B] or NULL
   uint32_t *mask;            // [B, words] or NULL
   int32_t *counts;           // [B] or NULL
+  int group_shift;           // log2 of the chunks of a thread's group (sample_kernel)
 };
 
 // Rows cut into S slices of `slice` tokens (a multiple of kStep8): what the
@@ -785,7 +788,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
   const bool want_m = mp > 0.f && !want_k && !want_p;  // min_p alone
   // (a row of one chunk per thread under min_p: the pass is as short as its groups, 2,000
   // tokens 10.5 us against 11.1)
-  const bool use_g = words <= kMaskWords && ((want_m && vocab > kStep8) || (want_k && topk <= kSampleThreads));
+  const bool use_g = (want_m && vocab > kStep8) || (want_k && topk <= kSampleThreads);
+  const int gsh = a.group_shift, gmask = (1 << gsh) - 1;
   const bool track = !want_k && !want_p && !use_g;
   float tmx = -INFINITY;
   int tmi = 0;
@@ -798,13 +802,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
       float gm = -INFINITY;
       for_chunks(Every{}, [&](const float v[kVec], int64_t) __attribute__((always_inline)) {
         gm = fmaxf(gm, max8(v));
-        if ((++c & (kGroup - 1)) == 0) {
-          gmax[c / kGroup - 1][tid] = gm;
+        if ((++c & gmask) == 0) {
+          gmax[(c >> gsh) - 1][tid] = gm;
           tmx = fmaxf(tmx, gm);
           gm = -INFINITY;
         }
       });
-      if (c & (kGroup - 1)) gmax[c / kGroup][tid] = gm;
+      if (c & gmask) gmax[c >> gsh][tid] = gm;
       tmx = fmaxf(tmx, gm);
     } else {
       for_chunks(Own{}, [&](const float v[kVec], int64_t) __attribute__((always_inline)) { tmx = fmaxf(tmx, max8(v)); });
@@ -911,9 +915,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
     const bool captured = mx < INFINITY && (want_m || bcap < kBins - 1);
     const float bcap1 = want_m ? INFINITY : static_cast<float>(bcap + 1);
     if (captured && use_g) {
-      // The groups whose maximum is in the range, four lanes (one chunk each) per group.
+      // The groups whose maximum is in the range, a lane per chunk.
       uint16_t *hits = reinterpret_cast<uint16_t *>(fmass);  // the top_p mass bins are not used with top_k or min_p
-      const int n_g = (vocab + kGroup * kStep8 - 1) / (kGroup * kStep8);
+      const int n_g = (((vocab + kStep8 - 1) / kStep8 - 1) >> gsh) + 1;
       for (int g = 0; g < n_g; ++g) {
         const float m = gmax[g][tid];
         const bool hit = order_key(m) >= key_lo && (mx - m) * kBinScale < bcap1;
@@ -928,10 +932,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
       }
       __syncthreads();
       const int nh = nhit;
-      if (!want_m || nh <= kMaxHits) {
-        for (int t = tid; t < kGroup * nh; t += kSampleThreads) {
-          const int h = hits[t / kGroup];
-          const int64_t base = static_cast<int64_t>(h / kSampleThreads * kGroup + t % kGroup) * kStep8 +
+      if (!want_m || nh << gsh <= kMaxHitChunks) {
+        for (int t = tid; t < nh << gsh; t += kSampleThreads) {
+          const int h = hits[t >> gsh];
+          const int64_t base = static_cast<int64_t>((h / kSampleThreads << gsh) + (t & gmask)) * kStep8 +
                                static_cast<int64_t>(h % kSampleThreads) * kVec;
           if (base >= vocab) continue;
           float v[kVec];
@@ -949,15 +953,14 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
         listed = n > 0 && n <= kCand;
       }
       __syncthreads();
-    } else if (captured) {
+    } else if (captured) {  // top_p alone
       unsigned long long tmass = 0;
       // The key test is one float compare when the threshold is a negative
       // float (NEG; see the fast final loop).
       const float thr = __uint_as_float(~key_lo);  // with NEG: the keep threshold as a float
-      // (one instance per mass flag and key test: a select on them would do both)
+      // (one instance per key test: a select on it would do both)
       bool over = false;
-      auto capture = [&](auto with_mass, auto neg) __attribute__((always_inline)) {
-        constexpr bool M = decltype(with_mass)::value;
+      auto capture = [&](auto neg) __attribute__((always_inline)) {
         constexpr bool NEG = decltype(neg)::value;
         for_chunks2(Own{}, [&](const float v[kVec], int64_t base) __attribute__((always_inline)) {
 #pragma unroll
@@ -965,15 +968,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
             const float d = (mx - v[j]) * kBinScale;
             const bool kept = NEG ? v[j] >= thr : order_key(v[j]) >= key_lo;
             unsigned long long m = 0;
-            if constexpr (M) {
-              if (kept && d < static_cast<float>(kMassBins)) m = fixed_mass(v[j], mx);
-              tmass += m;
-            }
+            if (kept && d < static_cast<float>(kMassBins)) m = fixed_mass(v[j], mx);
+            tmass += m;
             const bool take = kept && d < bcap1;
             auto count = [&] {
               const int bn = static_cast<int>(d);
               atomicAdd(&fcnt[bn], 1u);
-              if constexpr (M) atomicAdd(&fmass[bn], m);
+              atomicAdd(&fmass[bn], m);
             };
             if (!over)
               over = append_or(take, v[j], base + j, count);
@@ -982,22 +983,12 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
           }
         });
       };
-      const bool neg_thr = key_lo < 0x80000000u;
-      if (hmass) {
-        if (neg_thr)
-          capture(std::true_type{}, std::true_type{});
-        else
-          capture(std::true_type{}, std::false_type{});
-      } else {
-        if (neg_thr)
-          capture(std::false_type{}, std::true_type{});
-        else
-          capture(std::false_type{}, std::false_type{});
-      }
-      if (hmass) {
-        const unsigned long long wm = wave_sum_u64(tmass);
-        if (lane == 0) atomicAdd(&sel_n, wm);
-      }
+      if (key_lo < 0x80000000u)
+        capture(std::true_type{});
+      else
+        capture(std::false_type{});
+      const unsigned long long wm = wave_sum_u64(tmass);
+      if (lane == 0) atomicAdd(&sel_n, wm);
       __syncthreads();
       n = ncand;
       listed = n > 0 && n <= kCand;
@@ -1308,13 +1299,14 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
   } else if (track) {
     race.bi = kNoToken - 1;  // another thread has it
   }
-  if (listed && words <= kMaskWords) {
+  if (listed) {
     // Final step on the list, which holds every kept token: the kept mass in
     // fixed point (exact, so independent of the list's order), the draw, the
     // mask (assembled in LDS) and the support size.
     uint32_t *mbits = ubuf;
+    const int nw0 = words < kMaskWords ? words : kMaskWords;
     if (a.mask)
-      for (int wd = tid; wd < words; wd += kSampleThreads) mbits[wd] = 0u;
+      for (int wd = tid; wd < nw0; wd += kSampleThreads) mbits[wd] = 0u;
     __syncthreads();
     unsigned long long zf = 0;
     for (int i = tid; i < n; i += kSampleThreads) {
@@ -1324,13 +1316,27 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const T *__restr
       zf += fixed_mass(x, mx);
       ++cnt;
       race.run(x, t);
-      if (a.mask) atomicOr(&mbits[t >> 5], 1u << (t & 31));
+      if (a.mask && (t >> 5) < nw0) atomicOr(&mbits[t >> 5], 1u << (t & 31));
     }
     unsigned long long ztot;
     (void)block_exscan_u64(zf, red64, ztot);  // its barriers also complete the mask
     lz = static_cast<float>(log(static_cast<double>(ztot)) - 22.180709777918249);  // - ln 2^32
     if (a.mask)
-      for (int wd = tid; wd < words; wd += kSampleThreads) a.mask[static_cast<int64_t>(b) * words + wd] = mbits[wd];
+      for (int wd = tid; wd < nw0; wd += kSampleThreads) a.mask[static_cast<int64_t>(b) * words + wd] = mbits[wd];
+    if (a.mask && words > kMaskWords) {  // uniform: the mask's further words, kMaskWords at a time
+      for (int w0 = kMaskWords; w0 < words; w0 += kMaskWords) {
+        __syncthreads();
+        const int nw = words - w0 < kMaskWords ? words - w0 : kMaskWords;
+        for (int wd = tid; wd < nw; wd += kSampleThreads) mbits[wd] = 0u;
+        __syncthreads();
+        for (int i = tid; i < n; i += kSampleThreads) {
+          const int wd = (cidx[i] >> 5) - w0;
+          if (ckey[i] >= key_lo && wd >= 0 && wd < nw) atomicOr(&mbits[wd], 1u << (cidx[i] & 31));
+        }
+        __syncthreads();
+        for (int wd = tid; wd < nw; wd += kSampleThreads) a.mask[static_cast<int64_t>(b) * words + w0 + wd] = mbits[wd];
+      }
+    }
   } else {
     float z = 0.f;
     float *qx = reinterpret_cast<float *>(ubuf) + (tid >> 6) * kFastQueue;
@@ -1365,6 +1371,13 @@ static Slices sample_slices(int batch, int vocab) {
   if (chunks - per < kMinSliceGain) return s;
   s.S = (chunks + per - 1) / per;
   s.slice = per * kStep8;
+  return s;
+}
+
+// kGroupShift up to 262,144 tokens, one more for every doubling.
+static int sample_group_shift(int vocab) {
+  int s = kGroupShift;
+  while ((static_cast<int64_t>(kGroups) << s) * kStep8 < vocab) ++s;
   return s;
 }
 
@@ -1424,7 +1437,7 @@ extern "C" int wkv_sample(const void *logits, int32_t logits_dtype, int64_t row_
                           int64_t step, int64_t *out_tokens, float *out_logprobs, uint32_t *out_mask,
                           int32_t *out_counts, void *stream) {
   const SampleArgs a{temperature, top_k, top_p, min_p, repetition_penalty, seen_tokens, seeds, step,
-                     out_tokens, out_logprobs, out_mask, out_counts};
+                     out_tokens, out_logprobs, out_mask, out_counts, sample_group_shift(vocab)};
   return launch_sample(logits, logits_dtype, row_stride, batch, vocab, a, nullptr, 0, stream);
 }
 
@@ -1435,6 +1448,6 @@ extern "C" int wkv_sample_sliced(const void *logits, int32_t logits_dtype, int64
                                  uint32_t *out_mask, int32_t *out_counts, void *workspace, int64_t workspace_bytes,
                                  void *stream) {
   const SampleArgs a{temperature, top_k, top_p, min_p, repetition_penalty, seen_tokens, seeds, step,
-                     out_tokens, out_logprobs, out_mask, out_counts};
+                     out_tokens, out_logprobs, out_mask, out_counts, sample_group_shift(vocab)};
   return launch_sample(logits, logits_dtype, row_stride, batch, vocab, a, workspace, workspace_bytes, stream);
 }
