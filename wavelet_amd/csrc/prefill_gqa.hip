@@ -420,7 +420,12 @@ __global__ __launch_bounds__(64 * kPrefillWaves, 2) void prefill_gqa_kernel(Pref
     const PrefillGrid &pg = kernel_args.pg;
     // Eight sub-items (item, share r of its unit groups) run at a time, one per XCD.
     const int q = (id >> 3) / pg.by_inner, r = (id >> 3) - q * pg.by_inner.d;
-    const int oct = pg.mixed ? r : q, inner = pg.mixed ? q : r;
+    int oct = pg.mixed ? r : q;
+    const int inner = pg.mixed ? q : r;
+    if (pg.mixed && (pg.by_inner.d & 1) == 0) {  // an even number of them: each row of the turn begins one further
+      oct = r + q - q / pg.by_inner * pg.by_inner.d;
+      oct = oct >= pg.by_inner.d ? oct - pg.by_inner.d : oct;
+    }
     const int sub = 8 * oct + (id & 7);
     if (sub >= pg.n_sub) return;
     const int item = sub >> pg.log2R;
@@ -1103,7 +1108,13 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
   // as their keys no longer stay in its L2 together. (us, after another -> in
   // turn: two prompts of 2,048 at 14/2 heads 42.4 -> 38.0, four of 1,500 48.8 ->
   // 41.1, two of 1,000 at 32/8 42.7 -> 39.2; but 1,024 workgroups, 16 of 256,
-  // 38.8 -> 53.4.)
+  // 38.8 -> 53.4.) The dispatcher deals an XCD's workgroups to its 32 CUs in turn
+  // as well: an even number of sub-items would put each on the same few CUs
+  // every time, the longest's among them, so the rows of the turn are rotated
+  // (8 ragged prompts of 133-400 at 28/4 heads 23.9 -> 20.7, fp8 26.6 -> 22.4).
+  // Over 192 shapes of 9 to 160 items of 50 to 2,000 tokens the turn takes 0.947 of
+  // the time of one sub-item after another, 0.72 at best and 1.1 at worst (few ragged
+  // sequences whose last round of workgroups ends up uneven).
   const int n_oct = (pg.n_sub + 7) / 8;
   pg.mixed = n_oct > 1 && static_cast<int64_t>(8) * n_oct * pg.n_inner <= 3 * kPrefillCus;
   pg.by_inner = fast_div(pg.mixed ? n_oct : pg.n_inner);
