@@ -19,7 +19,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("kv_dtype", ["bf16", "fp8_e4m3"])
 @pytest.mark.parametrize("hq,hkv,d,qlens,ctx", [
     (14, 2, 64, [255, 64, 1, 33, 256, 200, 31, 100], 0),  # 256 groups of a tile's heads: a tile to itself
-    (14, 2, 64, [257, 64, 1, 33, 256, 200, 31, 100], 0),  # 288: packed across tiles
+    (14, 2, 64, [257, 64, 1, 33, 256, 200, 31, 100], 0),  # 288
+    (14, 2, 64, [512, 64, 1, 33, 256, 200, 31, 100], 0),  # 512
+    (14, 2, 64, [513, 64, 1, 33, 256, 200, 31, 100], 0),  # 544: packed across tiles
     (16, 8, 128, [256, 1, 90, 17], 48),
     (16, 8, 128, [257, 1, 90, 17], 48),
     (5, 1, 128, [289, 0, 128, 7] * 4, 20),
@@ -33,8 +35,8 @@ def test_both_sides_of_the_packing_bounds(cuda, hq, hkv, d, qlens, ctx, kv_dtype
 
 
 @pytest.mark.parametrize("kv_dtype", ["bf16", "fp8_e4m3"])
-@pytest.mark.parametrize("hq,hkv,d,n_seq,shared", [(14, 2, 64, 8, 0), (16, 8, 128, 4, 0), (5, 1, 128, 16, 0),
-                                                   (3, 3, 64, 1, 0), (14, 2, 64, 2, 24), (3, 1, 128, 2, 96),
+@pytest.mark.parametrize("hq,hkv,d,n_seq,shared", [(14, 2, 64, 8, 0), (14, 2, 64, 16, 0), (16, 8, 128, 4, 0),
+                                                   (5, 1, 128, 16, 0), (3, 3, 64, 1, 0), (14, 2, 64, 2, 24), (3, 1, 128, 2, 96),
                                                    (28, 4, 128, 2, 40)])
 def test_values_of_later_tiles_that_are_not_finite(cuda, hq, hkv, d, n_seq, shared, kv_dtype):
     """Infinite and NaN values from token 160 on (a block's and a query tile's first) leave the 160 queries

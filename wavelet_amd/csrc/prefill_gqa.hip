@@ -244,8 +244,10 @@ __device__ __forceinline__ PrefillLine prefill_prefix(int *pfx, int *red, const 
       if (4 * ug < r.units) c[k] = r.n_steps > 0 ? r.n_steps : 1;
     }
     sum += c[k];
-    mx = c[k] > mx ? c[k] : mx;
-    n += __popcll(__ballot(c[k] > 0));  // of the wave
+    if constexpr (STATS) {
+      mx = c[k] > mx ? c[k] : mx;
+      n += __popcll(__ballot(c[k] > 0));  // of the wave
+    }
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int incl = sum;
@@ -257,8 +259,10 @@ __device__ __forceinline__ PrefillLine prefill_prefix(int *pfx, int *red, const 
   if constexpr (STATS) mx = wave_reduce(mx, [](int a, int b) { return a > b ? a : b; });
   if (lane == 63) {
     red[wave] = incl;
-    red[kPrefillWaves + wave] = mx;
-    red[2 * kPrefillWaves + wave] = n;
+    if constexpr (STATS) {
+      red[kPrefillWaves + wave] = mx;
+      red[2 * kPrefillWaves + wave] = n;
+    }
   }
   __syncthreads();
   int base = incl - sum;
@@ -976,7 +980,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_merge_kernel(
     const float *__restrict__ sinks) {
   constexpr int PF = prefill_part_floats<D>();
   __shared__ int pfx[kPrefillEntries + 1];
-  __shared__ int red[3 * kPrefillWaves];
+  __shared__ int red[kPrefillWaves];
   const int by = *prefill_shared_by<D>(part, pg.W);  // (on its way while the prefix is formed)
   const int total = prefill_prefix<false>(pfx, red, cu_q, seq_lens, max_seq, pg).total;
   const int shared_by = __builtin_amdgcn_readfirstlane(by);
@@ -1077,14 +1081,19 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
     }
   }
   // At most one unit group per CU with a tile's units to themselves (made up to
-  // a multiple of four by units without a head): so, as the chip has room for
-  // them and no group then runs on to a later tile's keys nor its waves on
-  // keys that they do not see. Past that, packed: the idle waves cost more.
+  // a multiple of four by units without a head), or two where three waves in
+  // four or more then have a head: so, as the chip has room for them and no
+  // group then runs on to a later tile's keys nor its waves on keys that they do
+  // not see. Past that, packed: the idle waves cost more.
   // (us, packed -> not: one prompt of 512 at 16/8 heads bf16 20.9 -> 19.7, fp8
   // 23.0 -> 21.1; at 28/4 21.3 -> 20.6; 256 groups so, two prompts of 512 at 16/8
-  // 22.2 -> 21.0; but 512 groups, four prompts, 25.2 -> 28.5.)
+  // 22.2 -> 21.0; but 512 groups, four prompts, 25.2 -> 28.5. Over 26 to 38
+  // shapes of 257 to 512 groups so, the time not packed against packed: 14/2
+  // heads d=64 bf16 0.974, fp8 0.942; 28/4 bf16 0.984, fp8 0.996; but 16/8 1.018
+  // and 0.993.)
   const int64_t tile_ug = (G + 3) / 4;
-  if (pg.W == 0 && items * n_qt * tile_ug <= kPrefillCus) {
+  const int per_cu = G >= 3 * tile_ug ? 2 : 1;
+  if (pg.W == 0 && items * n_qt * tile_ug <= per_cu * kPrefillCus) {
     U = static_cast<int>(4 * tile_ug);
     pg.n_ug = static_cast<int>(n_qt * tile_ug);
   }
@@ -1112,7 +1121,7 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
   // as well: an even number of sub-items would put each on the same few CUs
   // every time, the longest's among them, so the rows of the turn are rotated
   // (8 ragged prompts of 133-400 at 28/4 heads 23.9 -> 20.7, fp8 26.6 -> 22.4).
-  // Over 192 shapes of 9 to 160 items of 50 to 2,000 tokens the turn takes 0.947 of
+  // Over 192 shapes of 9 to 240 items of 50 to 2,000 tokens the turn takes 0.947 of
   // the time of one sub-item after another, 0.72 at best and 1.1 at worst (few ragged
   // sequences whose last round of workgroups ends up uneven).
   const int n_oct = (pg.n_sub + 7) / 8;
