@@ -1125,7 +1125,11 @@ static PrefillGrid prefill_grid(int batch, int Hkv, int G, int D, bool fp8, int 
   // the time of one sub-item after another, 0.72 at best and 1.1 at worst (few ragged
   // sequences whose last round of workgroups ends up uneven).
   const int n_oct = (pg.n_sub + 7) / 8;
-  pg.mixed = n_oct > 1 && static_cast<int64_t>(8) * n_oct * pg.n_inner <= 3 * kPrefillCus;
+  // Prompts only: over cached contexts (more than an eighth) a chain's length
+  // follows its sequence, the turn leaves the longest's tiles for last and the
+  // XCD's keys outgrow its L2 (4 x 600 over 1,000-3,000 at 32/8 fp8 107.7 -> 134.6).
+  const bool prompts = static_cast<int64_t>(8) * max_query_len >= static_cast<int64_t>(7) * max_seq;
+  pg.mixed = prompts && n_oct > 1 && static_cast<int64_t>(8) * n_oct * pg.n_inner <= 3 * kPrefillCus;
   pg.by_inner = fast_div(pg.mixed ? n_oct : pg.n_inner);
   pg.by_Hkv = fast_div(Hkv);
   return pg;
